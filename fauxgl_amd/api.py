@@ -885,7 +885,7 @@ class Context:
         buf = (ctypes.c_uint8 * bound.value)()
         n = ctypes.c_int64()
         N.check(L.fgl_encode_png(self._ptr(), buf, bound.value, ctypes.byref(n)), self._ptr())
-        return bytes(buf[:n.value])
+        return ctypes.string_at(buf, n.value)
 
     def SavePNG(self, path):
         """SavePNG(path, Image()) (util.go:56-63)."""

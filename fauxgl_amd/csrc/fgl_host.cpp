@@ -162,6 +162,8 @@ struct fgl_ctx {
     ResolveTent4 rs_t4{};              // the tables as packed uniform 4x weights, when they are
     hipEvent_t xev = nullptr;          // orders another context's stream after this one
     DevBuf dpart, dimg;
+    DevBuf png;    // EncodePNG's workspace
+    HostBuf hpng;  // the encoded stream's size and checksums as the host reads them back
     uint32_t side_rec_cap = 0, side_vtx_cap = 0, pair_cap = 0;
     DrawCounters last{};
 
@@ -2448,9 +2450,6 @@ int fgl_mesh_load_obj(fgl_ctx *ctx, const char *text, int64_t size, fgl_mesh **o
 
 namespace {
 
-constexpr int32_t kPngChunk = 4096;                              // filtered bytes per deflate piece
-constexpr int32_t kPngCapWords = (9 * kPngChunk + 64) / 32 + 2;  // worst case: all 9-bit literals
-
 uint32_t crc_table_entry(uint32_t n) {
     uint32_t c = n;
     for (int k = 0; k < 8; k++) c = (c & 1) ? 0xEDB88320u ^ (c >> 1) : c >> 1;
@@ -2476,8 +2475,8 @@ void put_be32(uint8_t *p, uint32_t v) {
 
 int64_t png_bound(const fgl_ctx *c) {
     const int64_t n = (int64_t)c->H * ((int64_t)c->W * 4 + 1);
-    const int64_t pieces = (n + kPngChunk - 1) / kPngChunk;
-    return 8 + 25 + 8 + 2 + pieces * kPngCapWords * 4 + 2 + 4 + 4 + 12;
+    const int64_t pieces = (n + PNG_CHUNK - 1) / PNG_CHUNK;
+    return 8 + 25 + 8 + 2 + pieces * PNG_CAP_WORDS * 4 + 2 + 4 + 4 + 12;
 }
 
 }  // namespace
@@ -2502,54 +2501,45 @@ int fgl_encode_png(fgl_ctx *ctx, uint8_t *out, int64_t cap, int64_t *len) {
     int r = materialize(c, CB_COLOR);
     if (r) return r;
     const int32_t W = c->W, H = c->H;
-    DevBuf flag, stream, pieces, sizes, adl, offs, packed;
-    HIPCHK(c, flag.ensure(4));
-    HIPCHK(c, hipMemsetAsync(flag.p, 0, 4, c->stream));
+    // one workspace, kept with the context and sized for four bytes a pixel:
+    // result, pieces' records, offsets, filtered stream (whole pieces),
+    // pieces' words, packed stream
+    const int64_t np = ((int64_t)H * ((int64_t)W * 4 + 1) + PNG_CHUNK - 1) / PNG_CHUNK;
+    const size_t words_bytes = (size_t)np * PNG_CAP_WORDS * 4;
+    auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+    const size_t o_rec = 256, o_offs = o_rec + up((size_t)np * sizeof(PngPiece)), o_str = o_offs + up((size_t)np * 8),
+                 o_words = o_str + (size_t)np * PNG_CHUNK, o_pack = o_words + up(words_bytes);
+    HIPCHK(c, c->png.ensure(o_pack + words_bytes));
+    HIPCHK(c, c->hpng.ensure(sizeof(PngResult)));
+    uint8_t *ws = c->png.as<uint8_t>();
+    PngResult *res = reinterpret_cast<PngResult *>(ws);
+    PngPiece *rec = reinterpret_cast<PngPiece *>(ws + o_rec);
+    uint8_t *packed = ws + o_pack;
+    HIPCHK(c, hipMemsetAsync(res, 0, sizeof(PngResult), c->stream));
     if ((r = launch(c, "png_opaque", [&] {
-             return launch_png_opaque(c->color.as<uint32_t>(), (int64_t)W * H, flag.as<uint32_t>(), c->stream);
+             return launch_png_opaque(c->color.as<uint32_t>(), (int64_t)W * H, res, c->stream);
          })))
         return r;
-    uint32_t translucent = 0;
-    HIPCHK(c, hipMemcpyAsync(&translucent, flag.p, 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    const int32_t bpp = translucent ? 4 : 3;  // image/png: RGBA unless NRGBA.Opaque()
-    const int64_t n = (int64_t)H * ((int64_t)W * bpp + 1);
-    const int64_t np = (n + kPngChunk - 1) / kPngChunk;
-    HIPCHK(c, stream.ensure((size_t)n));
-    HIPCHK(c, pieces.ensure((size_t)np * kPngCapWords * 4));
-    HIPCHK(c, sizes.ensure((size_t)np * 4));
-    HIPCHK(c, adl.ensure((size_t)np * 8));
-    HIPCHK(c, offs.ensure((size_t)np * 8));
+    // image/png: RGBA unless NRGBA.Opaque(); the kernels read the flag
     if ((r = launch(c, "png_filter", [&] {
-             return launch_png_filter(c->color.as<uint32_t>(), W, H, bpp, stream.as<uint8_t>(), c->stream);
+             return launch_png_filter(c->color.as<uint32_t>(), W, H, res, ws + o_str, c->stream);
          })))
         return r;
     if ((r = launch(c, "png_deflate", [&] {
-             return launch_png_deflate(stream.as<uint8_t>(), n, kPngChunk, kPngCapWords, np, pieces.as<uint32_t>(),
-                                       sizes.as<uint32_t>(), adl.as<uint32_t>(), c->stream);
+             return launch_png_deflate(ws + o_str, W, H, res, np, reinterpret_cast<uint32_t *>(ws + o_words), rec,
+                                       c->stream);
          })))
         return r;
-    std::vector<uint32_t> hs((size_t)np), ha((size_t)np * 2);
-    HIPCHK(c, hipMemcpyAsync(hs.data(), sizes.p, (size_t)np * 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(ha.data(), adl.p, (size_t)np * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    std::vector<uint64_t> ho((size_t)np);
-    uint64_t total = 0;
-    uint32_t a = 1, b = 0;  // Adler-32 of the whole stream from the pieces'
-    for (int64_t k = 0; k < np; k++) {
-        ho[k] = total;
-        total += hs[k];
-        const uint64_t plen = (uint64_t)std::min<int64_t>(kPngChunk, n - k * kPngChunk);
-        b = (uint32_t)((b + (plen % 65521u) * a + ha[2 * k + 1]) % 65521u);
-        a = (uint32_t)((a + ha[2 * k]) % 65521u);
-    }
-    HIPCHK(c, packed.ensure((size_t)total));
-    HIPCHK(c, hipMemcpyAsync(offs.p, ho.data(), (size_t)np * 8, hipMemcpyHostToDevice, c->stream));
     if ((r = launch(c, "png_pack", [&] {
-             return launch_png_pack(pieces.as<uint32_t>(), sizes.as<uint32_t>(), offs.as<uint64_t>(), kPngCapWords, np,
-                                    packed.as<uint8_t>(), c->stream);
+             return launch_png_pack(reinterpret_cast<uint32_t *>(ws + o_words), rec, W, H, np, res,
+                                    reinterpret_cast<uint64_t *>(ws + o_offs), packed, c->stream);
          })))
         return r;
+    HIPCHK(c, hipMemcpyAsync(c->hpng.p, res, sizeof(PngResult), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, wait_stream(c->stream));
+    const PngResult pr = *c->hpng.as<PngResult>();
+    const int32_t bpp = pr.translucent ? 4 : 3;
+    const uint64_t total = pr.total;
     // signature, IHDR, then the IDAT chunk around the zlib stream, IEND
     uint8_t *p = out;
     static const uint8_t sig[8] = {0x89, 'P', 'N', 'G', 0x0D, 0x0A, 0x1A, 0x0A};
@@ -2570,12 +2560,14 @@ int fgl_encode_png(fgl_ctx *ctx, uint8_t *out, int64_t cap, int64_t *len) {
     uint8_t *z = p + 8;
     z[0] = 0x78;  // deflate, 32K window
     z[1] = 0x9C;  // default level, header check
-    HIPCHK(c, hipMemcpyAsync(z + 2, packed.p, (size_t)total, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipMemcpyAsync(z + 2, packed, (size_t)total, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     z[2 + total] = 0x03;  // final block: fixed codes, end of block only
     z[3 + total] = 0x00;
-    put_be32(z + 4 + total, (b << 16) | a);
-    put_be32(z + zlen, crc32_update(0, p + 4, (size_t)(4 + zlen)));
+    put_be32(z + 4 + total, pr.adler);
+    // the chunk's CRC: "IDAT" and the header, the packed stream, what follows
+    const uint32_t crc = ~png_crc_append(~crc32_update(0, p + 4, 6), pr.crc, total);
+    put_be32(z + zlen, crc32_update(crc, z + 2 + total, 6));
     p = z + zlen + 4;
     static const uint8_t iend[12] = {0, 0, 0, 0, 'I', 'E', 'N', 'D', 0xAE, 0x42, 0x60, 0x82};
     memcpy(p, iend, 12);

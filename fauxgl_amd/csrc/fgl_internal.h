@@ -262,12 +262,30 @@ int64_t ingest_parse_int(const char *s, size_t n);
 void ingest_fields(const char *a, const char *b, std::vector<std::pair<const char *, size_t>> &out);
 
 // PNG encode (fgl_png.hip)
-hipError_t launch_png_opaque(const uint32_t *color, int64_t n, uint32_t *flag, hipStream_t s);
-hipError_t launch_png_filter(const uint32_t *color, int32_t W, int32_t H, int32_t bpp, uint8_t *out, hipStream_t s);
-hipError_t launch_png_deflate(const uint8_t *stream, int64_t n, int32_t chunk, int32_t cap_words, int64_t npieces,
-                              uint32_t *out, uint32_t *sizes, uint32_t *adl, hipStream_t s);
-hipError_t launch_png_pack(const uint32_t *pieces, const uint32_t *sizes, const uint64_t *offs, int32_t cap_words,
-                           int64_t npieces, uint8_t *dst, hipStream_t s);
+constexpr int32_t PNG_CHUNK = 4096;                              // filtered bytes per deflate piece
+constexpr int32_t PNG_CAP_WORDS = (9 * PNG_CHUNK + 64) / 32 + 2;  // a piece's worst case: all 9-bit literals
+struct PngPiece {
+    uint32_t size;    // bytes of the finished piece
+    uint32_t sa, sb;  // Adler-32 parts of its filtered bytes
+    uint32_t crc;     // CRC-32 register its bytes leave from 0
+};
+struct PngResult {
+    uint32_t translucent;  // an alpha below 255: RGBA, else RGB
+    uint32_t adler;
+    uint32_t crc;          // CRC-32 register the packed stream leaves from 0
+    uint32_t pad;
+    uint64_t total;        // bytes of the packed stream
+};
+hipError_t launch_png_opaque(const uint32_t *color, int64_t n, PngResult *res, hipStream_t s);
+hipError_t launch_png_filter(const uint32_t *color, int32_t W, int32_t H, const PngResult *res, uint8_t *out,
+                             hipStream_t s);
+hipError_t launch_png_deflate(const uint8_t *stream, int32_t W, int32_t H, const PngResult *res, int64_t npieces,
+                              uint32_t *out, PngPiece *pieces, hipStream_t s);
+// the pieces back to back in dst, offs their offsets; res: the stream's size and checksums
+hipError_t launch_png_pack(const uint32_t *words, const PngPiece *pieces, int32_t W, int32_t H, int64_t npieces,
+                           PngResult *res, uint64_t *offs, uint8_t *dst, hipStream_t s);
+// CRC-32 register after n bytes whose register from 0 is raw, following state
+uint32_t png_crc_append(uint32_t state, uint32_t raw, uint64_t n);
 
 // mesh preparation (fgl_mesh.hip)
 hipError_t launch_mesh_first_nonzero(const double *pos, int64_t nprim, int32_t nv, int64_t *block_first,
