@@ -1618,7 +1618,7 @@ struct fgl_nn {
     int64_t nparam = 0;
     DevBuf p, g, m, v;                        // f32 master weights, gradient, Adam moments
     DevBuf wf[NN_LAYERS], wt[NN_LAYERS];      // bf16 forward / flipped-transposed copies
-    DevBuf feat, act[NN_LAYERS - 1], out, gout, dy[2], dwp, dbp, rtmp, lpart, range, dpart;
+    DevBuf feat, act[NN_LAYERS - 1], out, gout, dy[2], dwp, lpart, range, dpart;
     int64_t step = 0;
     int32_t H = 0, W = 0;
 };
@@ -1767,10 +1767,8 @@ int nn_backward(fgl_nn *nn, fgl_ctx *src, fgl_ctx *target, float *loss) {
     HIPCHK(c, nn->dy[0].ensure(px * NN_C * 2));
     HIPCHK(c, nn->dy[1].ensure(px * NN_C * 2));
     HIPCHK(c, nn->lpart.ensure(nlb * 4));
-    const int64_t nw = nn_dw_waves(H, W);
-    HIPCHK(c, nn->dwp.ensure((size_t)nw * 9 * NN_C * NN_C * 4));
-    HIPCHK(c, nn->dbp.ensure((size_t)nw * NN_C * 4));
-    HIPCHK(c, nn->rtmp.ensure((size_t)NN_REDUCE_SPLIT * 9 * NN_C * NN_C * 4));
+    const int64_t nparts = nn_dw_parts(H, W);
+    HIPCHK(c, nn->dwp.ensure((size_t)nparts * (size_t)nn->nparam * 4));
     if ((r = launch(c, "nn_loss", [&] {
              return launch_nn_loss(nn->out.as<float>(), src->color.as<uint32_t>(), target->color.as<uint32_t>(), H, W,
                                    nn->gout.as<uint16_t>(), nn->lpart.as<float>(), nlb, c->stream);
@@ -1781,17 +1779,7 @@ int nn_backward(fgl_nn *nn, fgl_ctx *src, fgl_ctx *target, float *loss) {
         const uint16_t *x = l == 0 ? nn->feat.as<uint16_t>() : nn->act[l - 1].as<uint16_t>();
         const int32_t ci = nn->cin[l], co = nn->cout[l];
         if ((r = launch(c, "nn_dw", [&] {
-                 return launch_nn_dw(x, ci, dy, co, H, W, nn->dwp.as<float>(), nn->dbp.as<float>(), c->stream);
-             })))
-            return r;
-        if ((r = launch(c, "nn_reduce", [&] {
-                 return launch_nn_reduce(nn->dwp.as<float>(), nw, 9LL * co * ci, nn->g.as<float>() + nn->woff[l],
-                                         nn->rtmp.as<float>(), c->stream);
-             })))
-            return r;
-        if ((r = launch(c, "nn_reduce", [&] {
-                 return launch_nn_reduce(nn->dbp.as<float>(), nw, co, nn->g.as<float>() + nn->boff[l],
-                                         nn->rtmp.as<float>(), c->stream);
+                 return launch_nn_dw(x, ci, dy, co, H, W, nn->dwp.as<float>() + nn->woff[l], nn->nparam, c->stream);
              })))
             return r;
         if (l == 0) break;
@@ -1803,6 +1791,11 @@ int nn_backward(fgl_nn *nn, fgl_ctx *src, fgl_ctx *target, float *loss) {
             return r;
         dy = dx;
     }
+    // each partial holds every parameter: one sum for all layers
+    if ((r = launch(c, "nn_reduce", [&] {
+             return launch_nn_reduce(nn->dwp.as<float>(), nparts, nn->nparam, nn->g.as<float>(), c->stream);
+         })))
+        return r;
     std::vector<float> lp(nlb);
     HIPCHK(c, hipMemcpyAsync(lp.data(), nn->lpart.p, nlb * 4, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));

@@ -242,8 +242,6 @@ hipError_t depth_scratch(int32_t device, double **ptr);
 constexpr int NN_C = 32;         // hidden channels (widest layer)
 constexpr int NN_FEAT_C = 16;    // input feature channels (8 used)
 constexpr int NN_OUT_C = 16;     // output channels (3 used)
-constexpr int NN_DW_ROWS = 32;   // rows of 16 pixels per weight-gradient wave
-constexpr int NN_REDUCE_SPLIT = 64;  // first-pass rows of the partial-sum reduction
 constexpr int NN_LAYERS = 6;
 
 hipError_t launch_nn_range(const double *partial, int32_t nblocks, double *range, hipStream_t s);
@@ -313,10 +311,12 @@ hipError_t launch_nn_conv2(int cin_a, int cout_b, int epi_b, const uint16_t *in,
                            const uint16_t *wb, const float *bb, int32_t H, int32_t W, void *out,
                            const uint32_t *color, const double *depth, const double *range, int32_t nrange,
                            hipStream_t s);
-int64_t nn_dw_waves(int32_t H, int32_t W);
+// a layer's gradient as nn_dw_parts partial sums of its weights and then its
+// bias, partial k at partial + k * stride; summed over k by launch_nn_reduce
+int64_t nn_dw_parts(int32_t H, int32_t W);
 hipError_t launch_nn_dw(const uint16_t *x, int32_t Cin, const uint16_t *dy, int32_t Cout, int32_t H, int32_t W,
-                        float *partial, float *bpartial, hipStream_t s);
-hipError_t launch_nn_reduce(const float *part, int64_t n, int64_t len, float *out, float *tmp, hipStream_t s);
+                        float *partial, int64_t stride, hipStream_t s);
+hipError_t launch_nn_reduce(const float *part, int64_t n, int64_t len, float *out, hipStream_t s);
 hipError_t launch_nn_loss(const float *out, const uint32_t *color, const uint32_t *target, int32_t H, int32_t W,
                           uint16_t *gout, float *lpart, int32_t nblocks, hipStream_t s);
 hipError_t launch_nn_adam(float *p, const float *g, float *m, float *v, int64_t n, float lr, float b1, float b2,

@@ -1009,82 +1009,198 @@ __global__ __launch_bounds__(512) void k_nn_stream(const uint32_t *color, const 
 
 // ---------------------------------------------------------------------------
 // weight gradient: dw[tap][co][ci] = sum over pixels p of
-// x[p + d(tap)][ci] * dy[p][co]; each wave sums NN_DW_ROWS rows of 16
-// pixels and writes its own partial (9 * Cout * Cin floats) plus the bias
-// gradient partial (Cout floats).
+// x[p + d(tap)][ci] * dy[p][co], and the bias gradient, the sum of dy.
+//
+// The contraction runs over pixels, but both operands hold a pixel's
+// channels contiguously: a row of DW_W pixels of each is staged in LDS as it
+// lies in memory and read back transposed (ds_read_b64_tr_b16: lane i of a
+// 16-lane group gets channel i of four pixels), so a tap's shift is a row
+// address.  A workgroup walks a band of rows of one DW_W-pixel strip, a wave
+// 32 pixels of each row: per step it reads one row of x at its three shifts
+// and one row of dy, whose fragments stay in registers for the three x rows
+// they meet.  The next rows are loaded from HBM before this row's MFMAs.
+// Every pixel order is a valid contraction order as long as both operands
+// use it, so the lane layout of the reads need only agree.
+//
+// What bounds it: HBM, reading x and dy once (265 MB for 32 x 32 channels at
+// 1920 x 1080).  Gathering both operands two bytes at a time from global
+// memory, one wave per 16 x 32 pixels, took 4.07 ms for the six layers, and
+// the reduction of its 4080 partials 0.28 ms; now 0.39 and 0.023 ms (71 us,
+// 3.7 TB/s, for 32 x 32 channels).
+constexpr int DW_W = 128;
+constexpr int DW_WG = 512;     // workgroups aimed at: two per CU, all resident
+constexpr int DW_MIN_ROWS = 8;  // rows of a band at least (a band reads two halo rows of x)
 
-__global__ __launch_bounds__(64) void k_nn_dw(const uint16_t *x, int32_t Cin, const uint16_t *dy, int32_t Cout,
-                                              int32_t H, int32_t W, float *partial, float *bpartial) {
-    const int lane = threadIdx.x;
-    const int x0 = blockIdx.x * 16;
-    const int y0 = blockIdx.y * NN_DW_ROWS;
-    const int pm = lane & 15, kg = lane >> 4;
-    const int64_t wave_id = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-    const int nco = Cout >> 4, nci = Cin >> 4;
-    float bsum = 0.0f;  // bias gradient for channel (co tile, pm) accumulated by kg == 0 lanes
-    for (int cot = 0; cot < nco; cot++) {
-        for (int cit = 0; cit < nci; cit++) {
-            f32x4 acc[9];
-#pragma unroll
-            for (int t = 0; t < 9; t++) acc[t] = f32x4{0, 0, 0, 0};
-            for (int r = 0; r < NN_DW_ROWS; r++) {
-                const int y = y0 + r;
-                if (y >= H) break;
-                // A = dy^T: row co = cot*16 + pm, k = pixels x0 + 4*kg + j
-                bf16x4 a;
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int px = x0 + 4 * kg + j;
-                    a[j] = px < W ? (short)dy[((int64_t)y * W + px) * Cout + cot * 16 + pm] : (short)0;
-                    if (cit == 0 && px < W) bsum += bf2f((uint16_t)a[j]);
-                }
-#pragma unroll
-                for (int tap = 0; tap < 9; tap++) {
-                    const int sy = y + tap / 3 - 1;
-                    bf16x4 b;
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const int px = x0 + 4 * kg + j;
-                        const int sx = px + tap % 3 - 1;
-                        const bool ok = px < W && sy >= 0 && sy < H && sx >= 0 && sx < W;
-                        b[j] = ok ? (short)x[((int64_t)sy * W + sx) * Cin + cit * 16 + pm] : (short)0;
-                    }
-                    acc[tap] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[tap], 0, 0, 0);
-                }
-            }
-            // lane holds rows co = cot*16 + 4*kg + j, column ci = cit*16 + pm
-            float *pw = partial + wave_id * 9 * Cout * Cin;
-#pragma unroll
-            for (int tap = 0; tap < 9; tap++)
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    pw[((int64_t)tap * Cout + cot * 16 + 4 * kg + j) * Cin + cit * 16 + pm] = acc[tap][j];
-        }
-        // bias: lanes with the same pm hold partial sums over their pixels
-        float s = bsum;
-        s += __shfl_xor(s, 16);
-        s += __shfl_xor(s, 32);
-        if (kg == 0) bpartial[wave_id * Cout + cot * 16 + pm] = s;
-        bsum = 0.0f;
-    }
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+// bytes of one staged pixel: 96 puts the eight pixels 32 lanes read into
+// eight different bank groups, 32 does as it is
+template <int C>
+struct DwStride {
+    static constexpr int v = C == 32 ? 96 : 32;
+};
+
+// channels c16 * 16 + (lane & 15) of 8 pixels: k = 8 * (lane >> 4) + j is
+// pixel 4 * (lane >> 4) + j (j < 4) or 16 + 4 * (lane >> 4) + j - 4
+template <int C>
+FGL_D bf16x8 dw_frag(const uint8_t *row, int pixel, int c16, int lane) {
+    typedef __attribute__((address_space(3))) i16x4 *lds_i16x4;
+    constexpr int S = DwStride<C>::v;
+    const uint8_t *q = row + (pixel + 4 * (lane >> 4) + ((lane & 15) >> 2)) * S + c16 * 32 + (lane & 3) * 8;
+    const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4)q);
+    const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4)(q + 16 * S));
+    typedef short i16x8 __attribute__((ext_vector_type(8)));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// out[k2][i] = sum over k = k2, k2 + ks, ... < n of part[k * len + i]
-// (grid: len / 256 x ks); a second pass with n = ks sums the ks rows
-__global__ void k_nn_reduce(const float *part, int64_t n, int64_t len, float *out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= len) return;
-    const int64_t ks = gridDim.y;
-    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
-    int64_t k = blockIdx.y;
-    for (; k + 3 * ks < n; k += 4 * ks) {
-        s0 += part[k * len + i];
-        s1 += part[(k + ks) * len + i];
-        s2 += part[(k + 2 * ks) * len + i];
-        s3 += part[(k + 3 * ks) * len + i];
+template <int CI, int CO>
+__global__ __launch_bounds__(256, 2) void k_nn_dw(const uint16_t *x, const uint16_t *dy, int32_t H, int32_t W,
+                                                  int32_t nstrips, int32_t band_h, float *partial, int64_t stride) {
+    constexpr int NI = CI / 16, NO = CO / 16;
+    constexpr int SX = DwStride<CI>::v, SY = DwStride<CO>::v;
+    constexpr int XPIX = DW_W + 2;
+    constexpr int XROW = XPIX * SX, YROW = DW_W * SY;
+    constexpr int XQ = XPIX * CI / 8, YQ = DW_W * CO / 8;  // 16-byte loads of a row
+    constexpr int XIT = (XQ + 255) / 256, YIT = (YQ + 255) / 256;
+    constexpr int TAPS = 3;  // taps summed over the waves at a time
+    constexpr int RED = 4 * TAPS * CO * CI * 4;
+    constexpr int STAGE = 2 * (XROW + YROW);
+    __shared__ __attribute__((aligned(16))) uint8_t lds[STAGE > RED ? STAGE : RED];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int x0 = (int)(blockIdx.x % (unsigned)nstrips) * DW_W, y0 = (int)(blockIdx.x / (unsigned)nstrips) * band_h;
+    const int y1 = y0 + band_h < H ? y0 + band_h : H;
+
+    // row r of x (pixels x0 - 1 .. x0 + DW_W) and row r + 1 of dy: clamped
+    // unconditional loads, zero outside the image and, for dy, the band
+    auto fetch = [&](int r, uint4 (&vx)[XIT], uint4 (&vy)[YIT]) {
+        const int cr = r < 0 ? 0 : (r >= H ? H - 1 : r);
+#pragma unroll
+        for (int it = 0; it < XIT; it++) {
+            const int q = tid + it * 256;
+            const int px = x0 - 1 + q / (CI / 8), c = q % (CI / 8);
+            const int cx = px < 0 ? 0 : (px >= W ? W - 1 : px);
+            if (it == 0 || q < XQ) vx[it] = *reinterpret_cast<const uint4 *>(x + ((int64_t)cr * W + cx) * CI + c * 8);
+            if (cx != px || cr != r) vx[it] = make_uint4(0, 0, 0, 0);
+        }
+        const int ry = r + 1, cy = ry < H ? ry : H - 1;
+#pragma unroll
+        for (int it = 0; it < YIT; it++) {
+            const int q = tid + it * 256;
+            const int px = x0 + q / (CO / 8), c = q % (CO / 8);
+            const int cx = px >= W ? W - 1 : px;
+            vy[it] = *reinterpret_cast<const uint4 *>(dy + ((int64_t)cy * W + cx) * CO + c * 8);
+            if (cx != px || ry >= y1) vy[it] = make_uint4(0, 0, 0, 0);
+        }
+    };
+    static_assert(XQ >= 256 && YQ % 256 == 0, "every thread has a first x load, all dy loads are whole");
+    auto put = [&](uint8_t *buf, const uint4 (&vx)[XIT], const uint4 (&vy)[YIT]) {
+#pragma unroll
+        for (int it = 0; it < XIT; it++) {
+            const int q = tid + it * 256;
+            if (q < XQ) *reinterpret_cast<uint4 *>(buf + (q / (CI / 8)) * SX + (q % (CI / 8)) * 16) = vx[it];
+        }
+#pragma unroll
+        for (int it = 0; it < YIT; it++) {
+            const int q = tid + it * 256;
+            *reinterpret_cast<uint4 *>(buf + XROW + (q / (CO / 8)) * SY + (q % (CO / 8)) * 16) = vy[it];
+        }
+    };
+
+    f32x4 acc[9][NO][NI], accb[NO];
+#pragma unroll
+    for (int o = 0; o < NO; o++) {
+        accb[o] = f32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int t = 0; t < 9; t++)
+#pragma unroll
+            for (int i = 0; i < NI; i++) acc[t][o][i] = f32x4{0, 0, 0, 0};
     }
-    for (; k < n; k += ks) s0 += part[k * len + i];
-    out[(int64_t)blockIdx.y * len + i] = (s0 + s1) + (s2 + s3);
+    bf16x8 d[3][NO], ones;  // dy rows r + 1, r, r - 1
+#pragma unroll
+    for (int k = 0; k < 8; k++) ones[k] = (__bf16)1.0f;
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int o = 0; o < NO; o++) d[k][o] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+
+    uint4 vx[XIT], vy[YIT];
+    fetch(y0 - 1, vx, vy);
+    int flip = 0;
+    for (int r = y0 - 1; r <= y1; r++, flip ^= 1) {
+        uint8_t *buf = lds + flip * (XROW + YROW);
+        put(buf, vx, vy);
+        if (r < y1) fetch(r + 1, vx, vy);
+        // one barrier a row: the buffer written next was last read before it
+        __syncthreads();
+#pragma unroll
+        for (int o = 0; o < NO; o++) {
+            d[2][o] = d[1][o];
+            d[1][o] = d[0][o];
+            d[0][o] = dw_frag<CO>(buf + XROW, wave * 32, o, lane);
+            accb[o] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d[0][o], ones, accb[o], 0, 0, 0);
+        }
+        if (r < 0 || r >= H) continue;  // a padding row
+#pragma unroll
+        for (int kx = 0; kx < 3; kx++)
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                const bf16x8 b = dw_frag<CI>(buf, wave * 32 + kx, i, lane);
+#pragma unroll
+                for (int ky = 0; ky < 3; ky++)
+#pragma unroll
+                    for (int o = 0; o < NO; o++)
+                        acc[3 * ky + kx][o][i] =
+                            __builtin_amdgcn_mfma_f32_16x16x32_bf16(d[ky][o], b, acc[3 * ky + kx][o][i], 0, 0, 0);
+            }
+    }
+
+    // the four waves' sums: lane (pm, g) holds rows co = 16 o + 4 g + j,
+    // column ci = 16 i + pm
+    float *red = reinterpret_cast<float *>(lds);
+    float *pw = partial + (int64_t)blockIdx.x * stride;
+    const int pm = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int t0 = 0; t0 < 9; t0 += TAPS) {
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TAPS; t++)
+#pragma unroll
+            for (int o = 0; o < NO; o++)
+#pragma unroll
+                for (int i = 0; i < NI; i++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        red[((wave * TAPS + t) * CO + 16 * o + 4 * g + j) * CI + 16 * i + pm] = acc[t0 + t][o][i][j];
+        __syncthreads();
+        constexpr int N = TAPS * CO * CI;
+        for (int q = tid; q < N; q += 256)
+            pw[t0 * CO * CI + q] = (red[q] + red[N + q]) + (red[2 * N + q] + red[3 * N + q]);
+    }
+    __syncthreads();
+    if (pm == 0)
+#pragma unroll
+        for (int o = 0; o < NO; o++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) red[wave * CO + 16 * o + 4 * g + j] = accb[o][j];
+    __syncthreads();
+    if (tid < CO) pw[9 * CO * CI + tid] = (red[tid] + red[CO + tid]) + (red[2 * CO + tid] + red[3 * CO + tid]);
+}
+
+// out[i] = sum over k < n of part[k * len + i]: 64 columns a workgroup, the
+// rows dealt over its four waves.
+__global__ __launch_bounds__(256) void k_nn_reduce(const float *part, int64_t n, int64_t len, float *out) {
+    __shared__ float s[4][64];
+    const int col = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t i = (int64_t)blockIdx.x * 64 + col;
+    const float *p = part + (i < len ? i : len - 1);
+    float a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    int64_t k = wave;
+    for (; k + 28 < n; k += 32)
+#pragma unroll
+        for (int u = 0; u < 8; u++) a[u] += p[(k + 4 * u) * len];
+    for (; k < n; k += 4) a[0] += p[k * len];
+    s[wave][col] = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+    __syncthreads();
+    if (wave == 0 && i < len) out[i] = (s[0][col] + s[1][col]) + (s[2][col] + s[3][col]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1233,18 +1349,33 @@ hipError_t launch_nn_stream(int epi, const uint32_t *color, const double *depth,
     return hipGetLastError();
     return hipGetLastError();
 }
-int64_t nn_dw_waves(int32_t H, int32_t W) { return (int64_t)((W + 15) / 16) * ((H + NN_DW_ROWS - 1) / NN_DW_ROWS); }
+// bands of rows such that strips x bands come near DW_WG, none of them
+// shorter than DW_MIN_ROWS
+static int32_t dw_band(int32_t H, int32_t W) {
+    const int64_t strips = (W + DW_W - 1) / DW_W;
+    const int64_t rows = (H * strips + DW_WG - 1) / DW_WG;
+    return (int32_t)(rows < DW_MIN_ROWS ? DW_MIN_ROWS : (rows > H ? H : rows));
+}
+int64_t nn_dw_parts(int32_t H, int32_t W) {
+    const int32_t band = dw_band(H, W);
+    return (int64_t)((W + DW_W - 1) / DW_W) * ((H + band - 1) / band);
+}
 hipError_t launch_nn_dw(const uint16_t *x, int32_t Cin, const uint16_t *dy, int32_t Cout, int32_t H, int32_t W,
-                        float *partial, float *bpartial, hipStream_t s) {
-    dim3 grid((W + 15) / 16, (H + NN_DW_ROWS - 1) / NN_DW_ROWS);
-    hipLaunchKernelGGL(k_nn_dw, grid, dim3(64), 0, s, x, Cin, dy, Cout, H, W, partial, bpartial);
+                        float *partial, int64_t stride, hipStream_t s) {
+    const int32_t strips = (W + DW_W - 1) / DW_W, band = dw_band(H, W);
+    const dim3 grid((unsigned)nn_dw_parts(H, W)), block(256);
+    if (Cin == 32 && Cout == 32)
+        hipLaunchKernelGGL((k_nn_dw<32, 32>), grid, block, 0, s, x, dy, H, W, strips, band, partial, stride);
+    else if (Cin == 16 && Cout == 32)
+        hipLaunchKernelGGL((k_nn_dw<16, 32>), grid, block, 0, s, x, dy, H, W, strips, band, partial, stride);
+    else if (Cin == 32 && Cout == 16)
+        hipLaunchKernelGGL((k_nn_dw<32, 16>), grid, block, 0, s, x, dy, H, W, strips, band, partial, stride);
+    else
+        return hipErrorInvalidValue;
     return hipGetLastError();
 }
-hipError_t launch_nn_reduce(const float *part, int64_t n, int64_t len, float *out, float *tmp, hipStream_t s) {
-    const int64_t ks = n < NN_REDUCE_SPLIT ? n : NN_REDUCE_SPLIT;
-    const unsigned gx = (unsigned)((len + 255) / 256);
-    hipLaunchKernelGGL(k_nn_reduce, dim3(gx, (unsigned)ks), dim3(256), 0, s, part, n, len, tmp);
-    hipLaunchKernelGGL(k_nn_reduce, dim3(gx, 1), dim3(256), 0, s, tmp, ks, len, out);
+hipError_t launch_nn_reduce(const float *part, int64_t n, int64_t len, float *out, hipStream_t s) {
+    hipLaunchKernelGGL(k_nn_reduce, dim3((unsigned)((len + 63) / 64)), dim3(256), 0, s, part, n, len, out);
     return hipGetLastError();
 }
 hipError_t launch_nn_loss(const float *out, const uint32_t *color, const uint32_t *target, int32_t H, int32_t W,
