@@ -624,7 +624,7 @@ int draw_buffers(fgl_ctx *c, DrawArgs &a) {
     HIPCHK(c, c->vals1.ensure((size_t)c->pair_cap * 4));
     a.nrsblocks = (int32_t)(((uint64_t)c->pair_cap + RS_BLOCK - 1) / RS_BLOCK);
     HIPCHK(c, c->hist.ensure((size_t)256 * a.nrsblocks * 4));
-    const size_t nsb = ((size_t)c->pair_cap + SPAN_THREADS - 1) / SPAN_THREADS + 1;
+    const size_t nsb = ((size_t)c->pair_cap + SPAN_THREADS - 1) / SPAN_THREADS * (SPAN_THREADS / SPAN_GROUP) + 1;
     HIPCHK(c, c->pspans.ensure((size_t)c->pair_cap * 4));
     HIPCHK(c, c->prows.ensure((size_t)c->pair_cap * 2));
     HIPCHK(c, c->span_bsum.ensure(nsb * 8));

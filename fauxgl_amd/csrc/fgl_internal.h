@@ -60,14 +60,14 @@ struct DrawArgs {
     // coverage spans
     uint32_t *pspans;           // spans per sorted pair
     uint16_t *prows;            // per sorted pair: its rows that have spans (ROWS_ALL: every row)
-    uint64_t *span_blocksum;    // per SPAN_THREADS pairs
+    uint64_t *span_blocksum;    // per SPAN_GROUP pairs
     uint64_t *span_blockoff;
     uint32_t *poff;             // first span of each sorted pair (pair_cap + 1 entries)
     Span *spans;
     uint32_t span_cap;
 
     // shaded fragments
-    uint64_t *frag_blocksum;    // fragments per SPAN_THREADS spans (accumulated by k_spans)
+    uint64_t *frag_blocksum;    // fragments per FRAG_BLOCK spans (accumulated by k_spans)
     uint64_t *frag_blockoff;    // offset of each span block within its group of 1024 blocks
     uint64_t *frag_gsum;        // fragments per group of 1024 span blocks
     uint32_t *foff;             // first fragment of each span (span_cap + 1 entries)
@@ -90,6 +90,7 @@ struct DrawArgs {
 
 constexpr int VS_THREADS = 256;
 constexpr int SPAN_THREADS = 256;
+constexpr int SPAN_GROUP = 64;  // pairs whose spans are placed together
 // Spans per fragment-count block: the shading kernel's waves each take one
 // such block (one span per lane) and need only its fragment offset.
 constexpr int FRAG_BLOCK = 64;
@@ -156,6 +157,7 @@ hipError_t launch_multi(int stage, const MultiArgs &m, uint32_t nblocks, const D
 uint32_t blocks_zero(const DrawArgs &a);
 uint32_t blocks_vs_deferred(const DrawArgs &a, bool many);
 uint32_t span_blocks(const DrawArgs &a);
+uint32_t spans_blocks(const DrawArgs &a, bool many);
 using MultiLaunch = hipError_t (*)(const MultiArgs &, uint32_t, const DrawArgs &, hipStream_t);
 hipError_t launch_zero_multi(const MultiArgs &m, uint32_t nb, const DrawArgs &rep, hipStream_t s);
 hipError_t launch_vs_multi(const MultiArgs &m, uint32_t nb, const DrawArgs &rep, hipStream_t s);

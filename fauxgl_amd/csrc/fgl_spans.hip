@@ -83,12 +83,11 @@ FGL_D uint32_t pair_spans(const DrawArgs &a, const uint32_t *keys, const uint32_
     return n > 0xffffffull ? 0xffffffu : (uint32_t)n;
 }
 
-// Spans per pair, summed per block of SPAN_THREADS pairs; also each tile's
-// range in the sorted pairs, and the zeroed fragment counts per span block
-// (the whole capacity, grid-wide) that k_spans accumulates into.
+// Spans per pair, summed per group of SPAN_GROUP pairs (a wave's); also each
+// tile's range in the sorted pairs, and the zeroed fragment counts per span
+// block (the whole capacity, grid-wide) that k_spans accumulates into.
 template <class G>
 FGL_D void span_count_body(const DrawArgs &a, const G &g) {
-    __shared__ uint64_t wsum[SPAN_THREADS / 64];
     if (a.ctr->overflow) return;
     const uint64_t nfb = ((uint64_t)a.span_cap + FRAG_BLOCK - 1) / FRAG_BLOCK;
     for (uint64_t k = (uint64_t)g.bid() * SPAN_THREADS + threadIdx.x; k < nfb; k += (uint64_t)g.nblk() * SPAN_THREADS)
@@ -109,24 +108,18 @@ FGL_D void span_count_body(const DrawArgs &a, const G &g) {
     }
     uint64_t v = n;
     for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
-    if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t s = 0;
-        for (int w = 0; w < SPAN_THREADS / 64; w++) s += wsum[w];
-        a.span_blocksum[g.bid()] = s;
-    }
+    if ((threadIdx.x & 63) == 0) a.span_blocksum[p / SPAN_GROUP] = v;
 }
 FGL_DRAW_KERNELS(k_span_count, span_count_body, __launch_bounds__(SPAN_THREADS))
 
-// Exclusive scan of the per-block span sums (one workgroup), total and
+// Exclusive scan of the per-group span sums (one workgroup), total and
 // capacity check.
 template <class G>
 FGL_D void span_scan_body(const DrawArgs &a, const G &) {
     __shared__ uint64_t lds[SCAN_THREADS / 64];
     if (a.ctr->overflow) return;
     const uint32_t E = a.ctr->npairs;
-    const int nb = (int)((E + SPAN_THREADS - 1) / SPAN_THREADS);
+    const int nb = (int)((E + SPAN_GROUP - 1) / SPAN_GROUP);
     const uint64_t total = scan_block_sums(a.span_blocksum, a.span_blockoff, nb, lds);
     if (threadIdx.x == SCAN_THREADS - 1) {
         if (total > a.span_cap) atomicOr(&a.ctr->overflow, 16u);
@@ -141,17 +134,6 @@ FGL_DRAW_KERNELS(k_span_scan, span_scan_body, __launch_bounds__(SCAN_THREADS))
 // edge(a, b, c) (context.go:147-149)
 FGL_D double edge(double ax, double ay, double bx, double by, double cx, double cy) {
     return (bx - cx) * (ay - cy) - (by - cy) * (ax - cx);
-}
-
-// Fragment counts per FRAG_BLOCK-span block: collected in LDS for the
-// FB_SLOTS blocks from the workgroup's first span on, in global memory
-// beyond that.
-constexpr uint32_t FB_SLOTS = 128;
-
-FGL_D void add_frags(const DrawArgs &a, uint32_t *lfb, uint32_t blk0, uint32_t blk, uint64_t cnt) {
-    if (!cnt) return;
-    if (blk - blk0 < FB_SLOTS) atomicAdd(&lfb[blk - blk0], (uint32_t)cnt);
-    else atomicAdd((unsigned long long *)&a.frag_blocksum[blk], (unsigned long long)cnt);
 }
 
 // Per-pair setup a wave shares through LDS: the edge values at the first
@@ -217,18 +199,29 @@ FGL_D void pair_setup(const DrawArgs &a, const uint32_t *keys, const uint32_t *v
 }
 
 // Span m of a pair (row yy = m / nk, wrapped column kk = m % nk, or the m-th
-// row pair_rows kept): the row's
-// edge values (yy row steps from ya), the skip to the first pixel that can
-// be inside, then the pixel walk of the reference's row loop
-// (context.go:185-221) through the tile's columns.  Returns the span and
-// its covered-pixel count.
+// row pair_rows kept): the row's edge values (yy row steps from ya), the skip
+// to the first pixel that can be inside, then the pixel walk of the
+// reference's row loop (context.go:185-221) through the tile's columns.
+// Returns the span and its covered-pixel count.
+//
+// The coordinates are finite (a record's box lies within BBOX_LIM), so each
+// edge value, the running sum of one step, is monotone along the row, and so
+// is the sign of its product with ra.  The pixels inside are therefore one
+// run, and left of the tile's columns the additions alone reach the same
+// values: a run that ended there leaves only pixels outside.  A wide
+// triangle's row is walked from its own start in every tile it crosses, so
+// that part was most of the kernel there (200,000-triangle soup at 1920x1080:
+// 0.67 ms with the tests made, 0.28 without them and with the shared groups
+// below).
 FGL_D Span pair_span(const PairSetup &q, uint32_t m, int32_t W, uint32_t &cnt_out) {
-    int32_t yy = (int32_t)(m / (uint32_t)q.nk), kk = (int32_t)(m % (uint32_t)q.nk);
+    int32_t yy = (int32_t)m, kk = 0;
     if (q.rows != ROWS_ALL) {  // the m-th kept row (nk == 1)
         uint32_t r = q.rows;
         for (uint32_t k = 0; k < m; k++) r &= r - 1;
         yy = __builtin_ctz(r);
-        kk = 0;
+    } else if (q.nk != 1) {
+        yy = (int32_t)(m / (uint32_t)q.nk);
+        kk = (int32_t)(m % (uint32_t)q.nk);
     }
     double w00 = q.w0, w01 = q.w1, w02 = q.w2;
     for (int32_t r = 0; r < yy; r++) {
@@ -245,13 +238,16 @@ FGL_D Span pair_span(const PairSetup &q, uint32_t m, int32_t W, uint32_t &cnt_ou
     if (w00 < 0 && d0 > d) d = d0;
     if (w01 < 0 && d1 > d) d = d1;
     if (w02 < 0 && d2 > d) d = d2;
-    d = (double)go_f2i(d);
-    if (d < 0) d = 0;
+    // int(d) and back; a d past int64 converts to its minimum, which the
+    // reference replaces by 0, and one past int32 lies right of the box
+    if (!(d < 9223372036854775808.0)) d = 0;
+    const bool far = d >= 2147483647.0;
+    const int32_t id = far ? 0 : (int32_t)d;
+    d = (double)id;
     double w0 = w00 + q.a12 * d;
     double w1 = w01 + q.a20 * d;
     double w2 = w02 + q.a01 * d;
-    const int64_t id = go_f2i(d);
-    const int32_t xs = (id > (int64_t)q.x1 - q.x0) ? q.x1 + 1 : q.x0 + (int32_t)id;
+    const int32_t xs = (far || id > q.x1 - q.x0) ? q.x1 + 1 : q.x0 + id;
     const int32_t k = q.kmin + kk;
     const int32_t kw = k * W;
     const int32_t pyk = y + k;
@@ -265,104 +261,141 @@ FGL_D Span pair_span(const PairSetup &q, uint32_t m, int32_t W, uint32_t &cnt_ou
     sp.pix = 0;
     sp.n = 0;
     uint32_t cnt = 0;
-    if (pyk >= q.cy0 && pyk <= q.cy1 && xa <= xb) {
-        bool was_inside = false;
-        for (int32_t x = xs; x <= xb; x++) {
-            const double b0 = w0 * q.ra, b1 = w1 * q.ra, b2 = w2 * q.ra;
-            if (b0 < 0 || b1 < 0 || b2 < 0) {
-                if (was_inside) break;
-            } else {
-                was_inside = true;
-                if (x >= xa) {
-                    if (cnt == 0) {
-                        sp.w[0] = w0;
-                        sp.w[1] = w1;
-                        sp.w[2] = w2;
-                        sp.pix = (uint16_t)((pyk - q.cy0) * TILE_W + (x - kw - q.cx0));
-                    }
-                    cnt++;
-                }
-            }
-            w0 += q.a12;
-            w1 += q.a20;
-            w2 += q.a01;
+    if (pyk >= q.cy0 && pyk <= q.cy1 && xa <= xb && xs <= xb) {
+        const double a12 = q.a12, a20 = q.a20, a01 = q.a01, ra = q.ra;
+        const int32_t left = xa - xs;  // pixels left of the tile
+#pragma unroll 8
+        for (int32_t j = 0; j < left; j++) {
+            w0 += a12;
+            w1 += a20;
+            w2 += a01;
         }
+        int32_t x = xs > xa ? xs : xa;
+        int32_t first = x;
+        for (; x <= xb; x++) {
+            // all three products before any branch: testing them one by one
+            // costs a third of the kernel (0.28 -> 0.40 ms on the soup)
+            const bool o0 = w0 * ra < 0, o1 = w1 * ra < 0, o2 = w2 * ra < 0;
+            const bool out = o0 || o1 || o2;
+            if (out && cnt) break;
+            if (!out) {
+                if (cnt == 0) {
+                    sp.w[0] = w0;
+                    sp.w[1] = w1;
+                    sp.w[2] = w2;
+                    first = x;
+                }
+                cnt++;
+            }
+            w0 += a12;
+            w1 += a20;
+            w2 += a01;
+        }
+        if (cnt) sp.pix = (uint16_t)((pyk - q.cy0) * TILE_W + (first - kw - q.cx0));
         sp.n = (uint16_t)(cnt | (k == 0 ? SPAN_INB : 0u));
     }
     cnt_out = cnt;
     return sp;
 }
 
-// One thread per pair sets up; then each wave writes its pairs' spans 64
-// at a time, one span per lane, so lanes share the walks evenly however
-// many rows each pair has.  A lane finds its span's pair as the shading
-// kernel finds a fragment's span (each pair marks its first span's window
-// position, a max-scan carries the mark) and reads the pair's setup from
-// LDS.  Also adds the covered pixels into the fragment count of each span
-// block it writes.
+// The spans of a group of SPAN_GROUP pairs, 64 at a time, one span per lane,
+// so lanes share the walks evenly however many rows each pair has, and the
+// covered pixels of each window added to the fragment counts of the (one or
+// two) FRAG_BLOCKs of the span list it lies in.  A lane finds its span's pair
+// as the shading kernel finds a fragment's span (each pair marks its first
+// span's window position, a max-scan carries the mark) and reads the pair's
+// setup from LDS.  The calling wave takes windows w0, w0 + dw, ...; n, excl:
+// its lane's pair's spans and their position in the group's T.
+FGL_D void group_windows(const DrawArgs &a, const PairSetup *setup, uint32_t *ostart, uint64_t gbase, uint32_t n,
+                         uint32_t excl, uint32_t T, uint32_t w0, uint32_t dw) {
+    const int lane = threadIdx.x & 63;
+    for (uint32_t base = w0 * 64; base < T; base += dw * 64) {
+        // the pair of the window's first span: the last pair that starts at
+        // or before it (pairs without spans start nowhere)
+        const uint64_t before = __ballot(n && excl <= base);
+        const uint32_t carry = 64u - (uint32_t)__builtin_clzll(before);
+        ostart[lane] = 0;
+        if (n && excl > base && excl - base < 64) ostart[excl - base] = (uint32_t)lane + 1;
+        __builtin_amdgcn_wave_barrier();
+        uint32_t om = wave_incl_max(ostart[lane]);
+        om = om ? om : carry;
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t q = base + (uint32_t)lane;
+        const int ow = (int)om - 1;
+        const uint32_t oexcl = __shfl(excl, ow);
+        const uint64_t blk = (gbase + base) / FRAG_BLOCK;
+        uint32_t cnt = 0;
+        if (q < T) {
+            const Span sp = pair_span(setup[ow], q - oexcl, a.W, cnt);
+            a.spans[gbase + q] = sp;
+        }
+        // both blocks' counts (at most 64 * 128 each) in one sum
+        if ((gbase + q) / FRAG_BLOCK != blk) cnt <<= 16;
+        const uint32_t both = wave_sum(cnt);
+        const uint32_t part = lane == 0 ? both & 0xffffu : both >> 16;
+        if (lane < 2 && part) atomicAdd((unsigned long long *)&a.frag_blocksum[blk + lane], (unsigned long long)part);
+    }
+}
+
+// Groups of SPAN_GROUP pairs, one pair per lane to set up.  A wave takes a
+// group to itself where there are many groups of few spans (the small
+// triangles of a dense mesh); where pairs average more than SPAN_SHARE spans,
+// or the groups are too few to fill the GPU, a workgroup's four waves share a
+// group's windows: a 12-triangle cube over four tiles has one group of 640
+// spans, which one wave alone took 33 us to walk (now 12; a sphere and a cube
+// at 512x512 95 -> 22 us).
+constexpr uint32_t SPAN_SHARE = 12;
+constexpr uint32_t SPAN_FEW = 2048;       // groups
+// Workgroups of a draw, each looping over the groups past the grid; a launch
+// for many draws gives each fewer, as most draws have few groups and every
+// block costs its dispatch.
+constexpr uint32_t SPANS_GRID_MAX = 16384, SPANS_GRID_MANY = 256;
+
 template <class G>
 FGL_D void spans_body(const DrawArgs &a, const G &g) {
-    __shared__ uint64_t wsum[SPAN_THREADS / 64];
-    __shared__ uint32_t lfb[FB_SLOTS];
     __shared__ uint32_t ostart[SPAN_THREADS / 64][64];
     __shared__ PairSetup setup[SPAN_THREADS / 64][64];
     if (a.ctr->overflow) return;
-    const uint32_t E = a.ctr->npairs;
+    const uint32_t E = a.ctr->npairs, NS = a.ctr->nspans;
+    const uint32_t ngroups = (E + SPAN_GROUP - 1) / SPAN_GROUP;
     const uint32_t *keys = a.keys[a.sorted_buf];
     const uint32_t *vals = a.vals[a.sorted_buf];
-    const uint32_t p = g.bid() * SPAN_THREADS + threadIdx.x;
-    const uint32_t n = p < E ? a.pspans[p] : 0u;
-    for (uint32_t k = threadIdx.x; k < FB_SLOTS; k += SPAN_THREADS) lfb[k] = 0;
-    // block-exclusive scan of n
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint64_t v = n;
-    for (int off = 1; off < 64; off <<= 1) {
-        uint64_t y = __shfl_up(v, off);
-        if (lane >= off) v += y;
-    }
-    if (lane == 63) wsum[wave] = v;
-    __syncthreads();
-    const uint64_t bbase = a.span_blockoff[g.bid()];
-    const uint32_t blk0 = (uint32_t)(bbase / FRAG_BLOCK);
-    uint64_t wbase = bbase;
-    for (int w = 0; w < wave; w++) wbase += wsum[w];
-    // this lane's pair's spans: [wbase + excl, wbase + excl + n)
-    const uint32_t excl = (uint32_t)(v - n);
-    const uint32_t T = (uint32_t)__shfl(v, 63);  // the wave's spans
-    if (p < E) a.poff[p] = (uint32_t)(wbase + excl);
-    if (n) pair_setup(a, keys, vals, p, setup[wave][lane]);
-    __builtin_amdgcn_wave_barrier();
-    Span *out = a.spans + wbase;
-    uint32_t carry = 0;  // pair lane + 1 of the last span of the previous window
-    for (uint32_t base = 0; base < T; base += 64) {
-        const uint32_t q = base + (uint32_t)lane;
-        ostart[wave][lane] = 0;
-        if (n && excl >= base && excl - base < 64) ostart[wave][excl - base] = (uint32_t)lane + 1;
-        __builtin_amdgcn_wave_barrier();
-        uint32_t om = wave_incl_max(ostart[wave][lane]);
-        om = om ? om : carry;
-        carry = __builtin_amdgcn_readlane(om, 63);
-        __builtin_amdgcn_wave_barrier();
-        const int ow = (int)om - 1 < 0 ? 0 : (int)om - 1;
-        const uint32_t oexcl = __shfl(excl, ow);
-        if (q < T) {
-            uint32_t cnt;
-            const Span sp = pair_span(setup[wave][ow], q - oexcl, a.W, cnt);
-            out[q] = sp;
-            if (cnt) {
-                const uint32_t blk = (uint32_t)((wbase + q) / FRAG_BLOCK);
-                add_frags(a, lfb, blk0, blk, cnt);
-            }
+    constexpr uint32_t WAVES = SPAN_THREADS / 64;
+    const bool share = ngroups <= SPAN_FEW || NS / SPAN_SHARE > E;
+    const uint32_t first = share ? g.bid() : g.bid() * WAVES + (uint32_t)wave;
+    const uint32_t step = share ? g.nblk() : g.nblk() * WAVES;
+    const int slot = share ? 0 : wave;
+    for (uint32_t grp = first; grp < ngroups; grp += step) {
+        const uint32_t p = grp * SPAN_GROUP + (uint32_t)lane;
+        const uint32_t n = p < E ? a.pspans[p] : 0u;
+        uint64_t v = n;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint64_t y = __shfl_up(v, off);
+            if (lane >= off) v += y;
         }
+        const uint64_t gbase = a.span_blockoff[grp];
+        const uint32_t excl = (uint32_t)(v - n);
+        const uint32_t T = (uint32_t)__shfl(v, 63);
+        if (!share || wave == 0) {
+            if (p < E) a.poff[p] = (uint32_t)(gbase + excl);
+            if (n) pair_setup(a, keys, vals, p, setup[slot][lane]);
+        }
+        if (share) __syncthreads();
+        else __builtin_amdgcn_wave_barrier();
+        group_windows(a, setup[slot], ostart[wave], gbase, n, excl, T, share ? (uint32_t)wave : 0u, share ? WAVES : 1u);
+        if (share) __syncthreads();  // the setups are read before the next group's are written
     }
-    __syncthreads();
-    for (uint32_t k = threadIdx.x; k < FB_SLOTS; k += SPAN_THREADS)
-        if (lfb[k]) atomicAdd((unsigned long long *)&a.frag_blocksum[blk0 + k], (unsigned long long)lfb[k]);
 }
 FGL_DRAW_KERNELS(k_spans, spans_body, __launch_bounds__(SPAN_THREADS))
 
 uint32_t span_blocks(const DrawArgs &a) {
     return (uint32_t)(((uint64_t)a.pair_cap + SPAN_THREADS - 1) / SPAN_THREADS);
+}
+uint32_t spans_blocks(const DrawArgs &a, bool many) {
+    const uint64_t groups = ((uint64_t)a.pair_cap + SPAN_GROUP - 1) / SPAN_GROUP;
+    const uint32_t most = many ? SPANS_GRID_MANY : SPANS_GRID_MAX;
+    return (uint32_t)(groups < most ? groups : most);
 }
 
 hipError_t launch_span_count(const DrawArgs &a, hipStream_t s) {
@@ -374,7 +407,7 @@ hipError_t launch_span_scan(const DrawArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 hipError_t launch_spans(const DrawArgs &a, hipStream_t s) {
-    hipLaunchKernelGGL(k_spans, dim3(span_blocks(a)), dim3(SPAN_THREADS), 0, s, a);
+    hipLaunchKernelGGL(k_spans, dim3(spans_blocks(a, false)), dim3(SPAN_THREADS), 0, s, a);
     return hipGetLastError();
 }
 hipError_t launch_span_count_multi(const MultiArgs &m, uint32_t nb, const DrawArgs &, hipStream_t s) {

@@ -900,7 +900,7 @@ uint32_t stage_blocks(int stage, const DrawArgs &a, bool many) {
         case ST_RADIX_SCATTER: return (uint32_t)a.nrsblocks;
         case ST_SPAN_COUNT: return span_blocks(a);
         case ST_SPAN_SCAN: return 1;
-        case ST_SPANS: return span_blocks(a);
+        case ST_SPANS: return spans_blocks(a, many);
         case ST_FRAG_SCAN: return frag_groups(a);
         case ST_SHADE: return span_grid(a);
         case ST_ROP: return (uint32_t)a.ntiles;
