@@ -435,6 +435,11 @@ def kernel_roofline(name, avg_ms, stats, W, H, ssaa, shader="phong"):
     elif name == "resolve":
         nbytes = 4 * npix + 4 * W * H
         unit_desc = f"4 B x {npix} source pixels + 4 B x {W * H} resolved pixels"
+    elif name == "zshade":
+        # shades only what its depth tests leave: bounded from below by the
+        # spans it reads and the pixels it writes
+        nbytes = 32 * stats["spans"] + 12 * npix
+        unit_desc = f"32 B x {stats['spans']} spans read + 12 B x {npix} pixels written"
     elif name == "spans":
         nbytes = 32 * stats["spans"] + 8 * stats["pairs"]
         unit_desc = f"32 B x {stats['spans']} spans + 8 B x {stats['pairs']} pairs"

@@ -18,10 +18,8 @@ namespace FGL_TILE_NS {
 template <class G>
 FGL_D void zero_body(const DrawArgs &a, const G &g) {
     int64_t i = (int64_t)g.bid() * blockDim.x + threadIdx.x;
-    if (i == 0) {
-        DrawCounters z = {};
-        *a.ctr = z;
-    }
+    static_assert(sizeof(DrawCounters) % 4 == 0 && sizeof(DrawCounters) / 4 <= 256, "one word a thread");
+    if (i < (int64_t)(sizeof(DrawCounters) / 4)) reinterpret_cast<uint32_t *>(a.ctr)[i] = 0;
     for (int64_t t = i; t < a.ntiles; t += (int64_t)g.nblk() * blockDim.x) {
         a.tstart[t] = 0;
         a.tend[t] = 0;

@@ -91,7 +91,7 @@ struct DevShader {
     double pw_yf;
     int32_t pw_frac, pw_big;
     int32_t pw_niter;  // bit length of pw_yi (squaring steps)
-    int32_t pw_pad;
+    int32_t tex_solid;  // the texture has no texel of alpha 0
     // For x in [pw_lo, pw_hi] every intermediate of the squaring loop, taken
     // without the frexp scaling, stays within 2^-1000 .. 2^1000.
     double pw_lo, pw_hi;
@@ -117,10 +117,13 @@ struct DrawCounters {
     uint32_t spans_lo, spans_hi; // unclamped span count
     uint32_t nfrags;             // fragments (clamped to capacity)
     uint32_t frags_lo, frags_hi; // unclamped fragment count
-    uint32_t pad2;
+    uint32_t zfirst;             // k_zshade draws (DrawArgs::zpick)
     // UpdatedPixels in UPD_PARTS partial sums (tile t adds into t % UPD_PARTS,
     // spreading the atomics over as many addresses); the host adds them up
     uint32_t upd[64];
+    // fragments in 64 partial sums (DrawArgs::zmode; span waves add into
+    // part wave % 64)
+    unsigned long long ftot[64];
 };
 constexpr int UPD_PARTS = 64;
 

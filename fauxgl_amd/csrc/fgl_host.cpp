@@ -118,6 +118,7 @@ hipError_t wait_stream(hipStream_t s) {
 struct Tex {
     void *d = nullptr;
     int32_t w = 0, h = 0, kind = 0;
+    bool solid = false;  // no texel of alpha 0
 };
 
 struct KStat {
@@ -152,7 +153,7 @@ struct fgl_ctx {
     DevBuf ctr, ntl, nrast, sstart, blocksum, blockoff, rec_main, tbox, side_rec, side_vtx;
     HostBuf hctr;  // the draw counters as the host reads them back
     DevBuf keys0, vals0, keys1, vals1, hist, dtot, tstart, tend, deferred;
-    DevBuf pspans, prows, span_bsum, span_boff, poff, spans;
+    DevBuf pspans, prows, span_bsum, span_boff, spans;
     DevBuf frag_bsum, frag_boff, frag_gsum, foff, frags;
     uint32_t span_cap = 0, frag_cap = 0;
     DevBuf in_pos, in_nrm, in_uv, in_col;
@@ -417,6 +418,7 @@ int fill_shader(fgl_ctx *c, const fgl_shader *sh, DevShader &d) {
         d.tex_w = it->second.w;
         d.tex_h = it->second.h;
         d.tex_pix = it->second.d;
+        d.tex_solid = it->second.solid;
     }
     return FGL_OK;
 }
@@ -537,6 +539,25 @@ void draw_setup(fgl_ctx *c, const fgl_state *st, const TileOps &T, int kind, con
     a.cbw = c->cbw;
 }
 
+// DrawArgs::zmode of a draw.  A fragment is Discard when its color is all
+// zero: a solid color is the shader's, a Phong color has the object color's
+// alpha (or, with a texture, the sample's), and a sample of a texture without
+// zero alphas has none either (its four weights are below 1 away from a texel
+// that lies in the texture; coordinates that are not finite give NaN).  Vertex
+// colors are not looked at.  Without a depth test every fragment survives, and
+// blended ones are shaded as they come.
+int draw_zmode(const DrawArgs &a) {
+    const DevShader &s = a.sh;
+    const double *c = s.kind == FGL_SHADER_SOLID ? s.color : s.obj;
+    const bool textured = s.has_tex != 0;
+    if (textured ? !s.tex_solid
+                 : s.kind == FGL_SHADER_SOLID ? (c[0] == 0 && c[1] == 0 && c[2] == 0 && c[3] == 0)
+                                              : (s.obj_is_discard || c[3] == 0))
+        return 0;
+    if (!a.st.write_color || !a.st.alpha_blend || (!textured && !(c[3] < 1))) return 1;
+    return a.st.read_depth ? 2 : 0;
+}
+
 // One pass of a draw: the kernel sequence on the context's stream.
 int draw_pass(fgl_ctx *c, const TileOps &T, const DrawArgs &a, int kind) {
     int r;
@@ -555,9 +576,11 @@ int draw_pass(fgl_ctx *c, const TileOps &T, const DrawArgs &a, int kind) {
     if ((r = launch(c, "span_count", [&] { return T.span_count(a, c->stream); }))) return r;
     if ((r = launch(c, "span_scan", [&] { return T.span_scan(a, c->stream); }))) return r;
     if ((r = launch(c, "spans", [&] { return T.spans(a, c->stream); }))) return r;
+    if (a.zmode && !a.zpick) return launch(c, "zshade", [&] { return T.zshade(a, c->stream); });
     if ((r = launch(c, "frag_scan", [&] { return T.frag_scan(a, c->stream); }))) return r;
     if ((r = launch(c, "shade", [&] { return T.shade(a, c->stream); }))) return r;
-    return launch(c, "rop", [&] { return T.rop(a, c->stream); });
+    if ((r = launch(c, "rop", [&] { return T.rop(a, c->stream); }))) return r;
+    return a.zpick ? launch(c, "zshade", [&] { return T.zshade(a, c->stream); }) : FGL_OK;
 }
 
 // The first part of a draw: checks, the shader, the framebuffer and state
@@ -579,6 +602,8 @@ int draw_begin(fgl_ctx *c, const fgl_state *st, const fgl_shader *sh, int kind, 
     }
     T = draw_ops(c, kind, in.n);
     draw_setup(c, st, *T, kind, in, a);
+    a.zmode = draw_zmode(a);
+    a.zpick = a.zmode && a.ntiles > ZTILES_DIRECT;
     const int64_t n = in.n;
 
     // starting capacities; grown on overflow
@@ -629,27 +654,29 @@ int draw_buffers(fgl_ctx *c, DrawArgs &a) {
     HIPCHK(c, c->prows.ensure((size_t)c->pair_cap * 2));
     HIPCHK(c, c->span_bsum.ensure(nsb * 8));
     HIPCHK(c, c->span_boff.ensure(nsb * 8));
-    HIPCHK(c, c->poff.ensure(((size_t)c->pair_cap + 1) * 4));
     HIPCHK(c, c->spans.ensure((size_t)c->span_cap * sizeof(Span)));
     a.pspans = c->pspans.as<uint32_t>();
     a.prows = c->prows.as<uint16_t>();
     a.span_blocksum = c->span_bsum.as<uint64_t>();
     a.span_blockoff = c->span_boff.as<uint64_t>();
-    a.poff = c->poff.as<uint32_t>();
     a.spans = c->spans.as<Span>();
     a.span_cap = c->span_cap;
     const size_t nfb = ((size_t)c->span_cap + FRAG_BLOCK - 1) / FRAG_BLOCK + 1;
-    HIPCHK(c, c->frag_bsum.ensure(nfb * 8));
-    HIPCHK(c, c->frag_boff.ensure(nfb * 8));
-    HIPCHK(c, c->frag_gsum.ensure((nfb / 1024 + 2) * 8));
-    HIPCHK(c, c->foff.ensure(((size_t)c->span_cap + 1) * 4));
-    HIPCHK(c, c->frags.ensure((size_t)c->frag_cap * sizeof(Frag)));
+    if (!a.zmode || a.zpick) {  // fragments that are tested first are not written out
+        HIPCHK(c, c->frag_bsum.ensure(nfb * 8));
+        HIPCHK(c, c->frag_boff.ensure(nfb * 8));
+        HIPCHK(c, c->frag_gsum.ensure((nfb / 1024 + 2) * 8));
+        HIPCHK(c, c->foff.ensure(((size_t)c->span_cap + 1) * 4));
+        HIPCHK(c, c->frags.ensure((size_t)c->frag_cap * sizeof(Frag)));
+    }
     a.frag_blocksum = c->frag_bsum.as<uint64_t>();
     a.frag_blockoff = c->frag_boff.as<uint64_t>();
     a.frag_gsum = c->frag_gsum.as<uint64_t>();
     a.foff = c->foff.as<uint32_t>();
     a.frags = c->frags.as<Frag>();
     a.frag_cap = c->frag_cap;
+    // past this many fragments run_draw would refuse to grow their buffer
+    a.frag_lim = std::max(c->frag_cap, (uint32_t)((0xfffff000ull - 65536) * 4 / 5));
 
     a.rec_main = c->rec_main.as<PrimRec>();
     a.tbox = c->tbox.as<int4>();
@@ -701,7 +728,7 @@ int run_draw(fgl_ctx *c, const fgl_state *st, const fgl_shader *sh, int kind, co
             if (f[1]) a.side_vtx_cap = std::min(a.side_vtx_cap, f[1]);
             if (f[2]) a.pair_cap = std::min(a.pair_cap, f[2]);
             if (f[3]) a.span_cap = std::min(a.span_cap, f[3]);
-            if (f[4]) a.frag_cap = std::min(a.frag_cap, f[4]);
+            if (f[4]) a.frag_cap = a.frag_lim = std::min(a.frag_cap, f[4]);
             std::memset(c->force_caps, 0, sizeof c->force_caps);
         }
 
@@ -914,6 +941,13 @@ int fgl_texture_create(fgl_ctx *ctx, int32_t width, int32_t height, int32_t kind
     t.w = width;
     t.h = height;
     t.kind = kind;
+    t.solid = true;
+    const size_t ntexel = (size_t)width * height;
+    if (kind == FGL_TEX_RGBA16) {
+        for (size_t k = 0; k < ntexel && t.solid; k++) t.solid = static_cast<const uint16_t *>(texels)[4 * k + 3] != 0;
+    } else {
+        for (size_t k = 0; k < ntexel && t.solid; k++) t.solid = static_cast<const uint8_t *>(texels)[4 * k + 3] != 0;
+    }
     HIPCHK(ctx, hipSetDevice(ctx->device));
     HIPCHK(ctx, hipMalloc(&t.d, bytes));
     hipError_t e = hipMemcpy(t.d, texels, bytes, hipMemcpyHostToDevice);
@@ -2817,9 +2851,10 @@ int batch_record_multi(fgl_batch *b) {
     struct Key {
         int round;
         const TileOps *T;
-        int kind, wire, shk, tex;
+        int kind, wire, shk, tex, zmode, zpick, wc;
         bool operator<(const Key &o) const {
-            return std::tie(round, T, kind, wire, shk, tex) < std::tie(o.round, o.T, o.kind, o.wire, o.shk, o.tex);
+            return std::tie(round, T, kind, wire, shk, tex, zmode, zpick, wc) <
+                   std::tie(o.round, o.T, o.kind, o.wire, o.shk, o.tex, o.zmode, o.zpick, o.wc);
         }
     };
     std::map<Key, size_t> gid;
@@ -2832,7 +2867,8 @@ int batch_record_multi(fgl_batch *b) {
         for (size_t k = 0; k < items.size(); k++) {
             const Item &it = items[k];
             if (it.round != rd) continue;
-            const Key key{rd, it.T, it.kind, it.a.st.wireframe ? 1 : 0, it.a.sh.kind, it.a.sh.has_tex ? 1 : 0};
+            const Key key{rd, it.T, it.kind, it.a.st.wireframe ? 1 : 0, it.a.sh.kind, it.a.sh.has_tex ? 1 : 0,
+                          it.a.zmode, it.a.zpick, it.a.st.write_color};
             auto f = gid.find(key);
             if (f == gid.end()) {
                 f = gid.emplace(key, members.size()).first;
@@ -2901,9 +2937,13 @@ int batch_record_multi(fgl_batch *b) {
         add(ST_SPAN_COUNT, 0);
         add(ST_SPAN_SCAN, 0);
         add(ST_SPANS, 0);
-        add(ST_FRAG_SCAN, 0);
-        add(ST_SHADE, 0);
-        add(ST_ROP, 0);
+        const bool zpick = keys[g].zpick != 0;
+        if (!G.rep.zmode || zpick) {
+            add(ST_FRAG_SCAN, 0);
+            add(ST_SHADE, 0);
+            add(ST_ROP, 0);
+        }
+        if (G.rep.zmode) add(ST_ZSHADE, 0);
         groups.push_back(std::move(G));
     }
     // each round's counters, gathered into the per-view slots

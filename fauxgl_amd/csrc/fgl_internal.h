@@ -54,7 +54,7 @@ struct DrawArgs {
     uint32_t *dtot;        // per-digit totals of the current radix pass
     int32_t nrsblocks;
     int32_t key_bits;
-    uint32_t *tstart, *tend;  // per tile range in the sorted pairs
+    uint32_t *tstart, *tend;  // per tile range of its spans
     int32_t sorted_buf;    // which of keys/vals holds the sorted result
 
     // coverage spans
@@ -62,7 +62,6 @@ struct DrawArgs {
     uint16_t *prows;            // per sorted pair: its rows that have spans (ROWS_ALL: every row)
     uint64_t *span_blocksum;    // per SPAN_GROUP pairs
     uint64_t *span_blockoff;
-    uint32_t *poff;             // first span of each sorted pair (pair_cap + 1 entries)
     Span *spans;
     uint32_t span_cap;
 
@@ -73,6 +72,13 @@ struct DrawArgs {
     uint32_t *foff;             // first fragment of each span (span_cap + 1 entries)
     Frag *frags;
     uint32_t frag_cap;
+
+    // How the fragments are drawn: 0 shaded, then tested and written in order
+    // (k_shade, k_rop); where no fragment can be Discard, tested first
+    // (k_zshade): 1 every color replaces the pixel's, 2 some may blend.
+    // zpick: the device picks one or the other by the draw's fragments.
+    int32_t zmode, zpick;
+    uint32_t frag_lim;          // fragments k_zshade draws at most (it stores none)
 
     // framebuffer and deferred clears
     uint32_t *color;       // NRGBA8 as little-endian u32
@@ -89,6 +95,9 @@ struct DrawArgs {
 };
 
 constexpr int VS_THREADS = 256;
+// Tiles up to which a draw that can be tested first is (see k_zshade): a
+// 1080p frame's, about two rounds of resident workgroups.
+constexpr int ZTILES_DIRECT = 2304;
 constexpr int SPAN_THREADS = 256;
 constexpr int SPAN_GROUP = 64;  // pairs whose spans are placed together
 // Spans per fragment-count block: the shading kernel's waves each take one
@@ -114,6 +123,7 @@ enum DrawStage : int {
     ST_FRAG_SCAN,
     ST_SHADE,
     ST_ROP,
+    ST_ZSHADE,  // in the place of the three before it, or after them (DrawArgs::zmode, zpick)
     ST_COUNT
 };
 
@@ -147,6 +157,7 @@ hipError_t launch_spans(const DrawArgs &a, hipStream_t s);
 hipError_t launch_frag_scan(const DrawArgs &a, hipStream_t s);
 hipError_t launch_shade(const DrawArgs &a, hipStream_t s);
 hipError_t launch_tile(const DrawArgs &a, hipStream_t s);
+hipError_t launch_zshade(const DrawArgs &a, hipStream_t s);
 // workgroups of one stage's launch for draw a (radix stages: per pass);
 // `many`: the launch covers many draws
 uint32_t stage_blocks(int stage, const DrawArgs &a, bool many);
@@ -182,7 +193,7 @@ struct TileOps {
     PassLaunch radix_hist;
     DrawLaunch radix_scan;
     PassLaunch radix_scatter;
-    DrawLaunch span_count, span_scan, spans, frag_scan, shade, rop;
+    DrawLaunch span_count, span_scan, spans, frag_scan, shade, rop, zshade;
     uint32_t (*stage_blocks)(int stage, const DrawArgs &a, bool many);
     hipError_t (*multi)(int stage, const MultiArgs &m, uint32_t nblocks, const DrawArgs &rep, hipStream_t s);
 };

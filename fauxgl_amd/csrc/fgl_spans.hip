@@ -83,13 +83,13 @@ FGL_D uint32_t pair_spans(const DrawArgs &a, const uint32_t *keys, const uint32_
     return n > 0xffffffull ? 0xffffffu : (uint32_t)n;
 }
 
-// Spans per pair, summed per group of SPAN_GROUP pairs (a wave's); also each
-// tile's range in the sorted pairs, and the zeroed fragment counts per span
-// block (the whole capacity, grid-wide) that k_spans accumulates into.
+// Spans per pair, summed per group of SPAN_GROUP pairs (a wave's); also the
+// zeroed fragment counts per span block (the whole capacity, grid-wide) that
+// k_spans accumulates into where the fragments are written out.
 template <class G>
 FGL_D void span_count_body(const DrawArgs &a, const G &g) {
     if (a.ctr->overflow) return;
-    const uint64_t nfb = ((uint64_t)a.span_cap + FRAG_BLOCK - 1) / FRAG_BLOCK;
+    const uint64_t nfb = a.zmode && !a.zpick ? 0 : ((uint64_t)a.span_cap + FRAG_BLOCK - 1) / FRAG_BLOCK;
     for (uint64_t k = (uint64_t)g.bid() * SPAN_THREADS + threadIdx.x; k < nfb; k += (uint64_t)g.nblk() * SPAN_THREADS)
         a.frag_blocksum[k] = 0;
     const uint32_t E = a.ctr->npairs;
@@ -101,10 +101,6 @@ FGL_D void span_count_body(const DrawArgs &a, const G &g) {
     if (p < E) {
         a.pspans[p] = n;
         a.prows[p] = rows;
-        // the tile's [start, end) in the sorted pairs
-        const uint32_t t = keys[p];
-        if (p == 0 || keys[p - 1] != t) a.tstart[t] = p;
-        if (p + 1 == E || keys[p + 1] != t) a.tend[t] = p + 1;
     }
     uint64_t v = n;
     for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
@@ -126,7 +122,6 @@ FGL_D void span_scan_body(const DrawArgs &a, const G &) {
         a.ctr->nspans = total > a.span_cap ? a.span_cap : (uint32_t)total;
         a.ctr->spans_lo = (uint32_t)total;
         a.ctr->spans_hi = (uint32_t)(total >> 32);
-        a.poff[E] = total > a.span_cap ? a.span_cap : (uint32_t)total;
     }
 }
 FGL_DRAW_KERNELS(k_span_scan, span_scan_body, __launch_bounds__(SCAN_THREADS))
@@ -305,9 +300,11 @@ FGL_D Span pair_span(const PairSetup &q, uint32_t m, int32_t W, uint32_t &cnt_ou
 // as the shading kernel finds a fragment's span (each pair marks its first
 // span's window position, a max-scan carries the mark) and reads the pair's
 // setup from LDS.  The calling wave takes windows w0, w0 + dw, ...; n, excl:
-// its lane's pair's spans and their position in the group's T.
+// its lane's pair's spans and their position in the group's T.  Where no
+// fragments are written out (zmode) the counts are summed in *frags instead
+// (zpick: too).
 FGL_D void group_windows(const DrawArgs &a, const PairSetup *setup, uint32_t *ostart, uint64_t gbase, uint32_t n,
-                         uint32_t excl, uint32_t T, uint32_t w0, uint32_t dw) {
+                         uint32_t excl, uint32_t T, uint32_t w0, uint32_t dw, uint64_t *frags) {
     const int lane = threadIdx.x & 63;
     for (uint32_t base = w0 * 64; base < T; base += dw * 64) {
         // the pair of the window's first span: the last pair that starts at
@@ -332,6 +329,10 @@ FGL_D void group_windows(const DrawArgs &a, const PairSetup *setup, uint32_t *os
         // both blocks' counts (at most 64 * 128 each) in one sum
         if ((gbase + q) / FRAG_BLOCK != blk) cnt <<= 16;
         const uint32_t both = wave_sum(cnt);
+        if (a.zmode) {
+            *frags += (both & 0xffffu) + (both >> 16);
+            if (!a.zpick) continue;
+        }
         const uint32_t part = lane == 0 ? both & 0xffffu : both >> 16;
         if (lane < 2 && part) atomicAdd((unsigned long long *)&a.frag_blocksum[blk + lane], (unsigned long long)part);
     }
@@ -366,6 +367,7 @@ FGL_D void spans_body(const DrawArgs &a, const G &g) {
     const uint32_t first = share ? g.bid() : g.bid() * WAVES + (uint32_t)wave;
     const uint32_t step = share ? g.nblk() : g.nblk() * WAVES;
     const int slot = share ? 0 : wave;
+    uint64_t frags = 0;
     for (uint32_t grp = first; grp < ngroups; grp += step) {
         const uint32_t p = grp * SPAN_GROUP + (uint32_t)lane;
         const uint32_t n = p < E ? a.pspans[p] : 0u;
@@ -378,14 +380,21 @@ FGL_D void spans_body(const DrawArgs &a, const G &g) {
         const uint32_t excl = (uint32_t)(v - n);
         const uint32_t T = (uint32_t)__shfl(v, 63);
         if (!share || wave == 0) {
-            if (p < E) a.poff[p] = (uint32_t)(gbase + excl);
+            if (p < E) {
+                // the first and the last pair of a tile bound its spans
+                const uint32_t t = keys[p];
+                if (p == 0 || keys[p - 1] != t) a.tstart[t] = (uint32_t)(gbase + excl);
+                if (p + 1 == E || keys[p + 1] != t) a.tend[t] = (uint32_t)(gbase + excl) + n;
+            }
             if (n) pair_setup(a, keys, vals, p, setup[slot][lane]);
         }
         if (share) __syncthreads();
         else __builtin_amdgcn_wave_barrier();
-        group_windows(a, setup[slot], ostart[wave], gbase, n, excl, T, share ? (uint32_t)wave : 0u, share ? WAVES : 1u);
+        group_windows(a, setup[slot], ostart[wave], gbase, n, excl, T, share ? (uint32_t)wave : 0u, share ? WAVES : 1u,
+                      &frags);
         if (share) __syncthreads();  // the setups are read before the next group's are written
     }
+    if (frags && lane == 0) atomicAdd(&a.ctr->ftot[(g.bid() * WAVES + (uint32_t)wave) % 64], (unsigned long long)frags);
 }
 FGL_DRAW_KERNELS(k_spans, spans_body, __launch_bounds__(SPAN_THREADS))
 

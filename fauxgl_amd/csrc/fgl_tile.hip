@@ -367,6 +367,15 @@ template <class G>
 FGL_D void frag_scan_body(const DrawArgs &a, const G &grid) {
     __shared__ uint64_t wsum[FRAG_GROUP / 64];
     if (a.ctr->overflow) return;
+    if (a.zpick) {
+        // depth first, or not: two fragments a pixel (see k_zshade)
+        const int l = threadIdx.x & 63;
+        uint64_t all = a.ctr->ftot[l];
+        for (int off = 32; off > 0; off >>= 1) all += __shfl_xor(all, off);
+        const bool zfirst = all >= 2ull * (uint64_t)a.W * (uint64_t)a.H;
+        if (grid.bid() == 0 && threadIdx.x == 0) a.ctr->zfirst = zfirst ? 1u : 0u;
+        if (zfirst) return;
+    }
     const uint32_t NS = a.ctr->nspans;
     const uint32_t nb = (NS + FRAG_BLOCK - 1) / FRAG_BLOCK;
     const uint32_t g = grid.bid();
@@ -534,7 +543,7 @@ FGL_D void shade_body(const DrawArgs &a, const G &grid) {
     __shared__ double slots[SPAN_THREADS / 64][SHADE_SLOTS][L::N];
     __shared__ uint64_t gpre[FRAG_GTAB];  // exclusive prefix of the group sums
     __shared__ uint64_t gw[SPAN_THREADS / 64];
-    if (a.ctr->overflow) return;
+    if (a.ctr->overflow || a.ctr->zfirst) return;
     const uint32_t NS = a.ctr->nspans;
     const uint32_t nb = (NS + FRAG_BLOCK - 1) / FRAG_BLOCK;
     const uint32_t ngroups = (nb + FRAG_GROUP - 1) / FRAG_GROUP;
@@ -701,15 +710,15 @@ FGL_D void rop_body(const DrawArgs &a, const G &g) {
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int t = (int)g.bid();
-    if (a.ctr->overflow) return;  // the host reruns the whole draw
+    if (a.ctr->overflow || a.ctr->zfirst) return;  // the host reruns the whole draw, or k_zshade draws it
     __shared__ uint32_t upd[TILE_THREADS / 64];
     const int tx = t % a.ntx, ty = t / a.ntx;
     const int cx0 = tx * TILE_W, cy0 = ty * TILE_H;
     const int cw = min(TILE_W, a.W - cx0), chh = min(TILE_H, a.H - cy0);
-    // the tile's fragment range [foff[poff[tstart]], foff[poff[tend]])
-    const uint32_t ps = a.tstart[t], pe = a.tend[t];
-    const uint32_t f0 = pe > ps ? a.foff[a.poff[ps]] : 0u;
-    const uint32_t f1 = pe > ps ? a.foff[a.poff[pe]] : 0u;
+    // the fragments of the tile's spans
+    const uint32_t s0 = a.tstart[t], s1 = a.tend[t];
+    const uint32_t f0 = s1 > s0 ? a.foff[s0] : 0u;
+    const uint32_t f1 = s1 > s0 ? a.foff[s1] : 0u;
     // the tile's blocks of deferred clears (CB_W x CB_H pixels each)
     constexpr int TBW = TILE_W / CB_W, TBH = TILE_H / CB_H;
     static_assert(TILE_W % CB_W == 0 && TILE_H % CB_H == 0, "tiles are whole clear blocks");
@@ -835,6 +844,440 @@ FGL_DRAW_KERNELS(k_rop, rop_body, __launch_bounds__(TILE_THREADS, FGL_ROP_WAVES)
 
 
 // ---------------------------------------------------------------------------
+// depth first, then shading, one workgroup per tile
+//
+// Where no fragment can be Discard (DrawArgs::zmode; the host checks the
+// shader's color, object color or texture), which fragments update the
+// framebuffer depends on their depths alone.  k_zshade runs the tile's depth
+// tests from the spans, in submission order and by the rounds k_rop uses, and
+// shades only what survives: with opaque colors each pixel's last survivor,
+// after the tests; with blending every survivor, through a queue in LDS from
+// which they are shaded a workgroup at a time and blended in order.  Nothing
+// is written but the framebuffer.  (Shading every fragment first wrote and
+// read back 16 bytes for each and shaded the 86% of the textured soup's 48
+// million that its depth tests reject.)
+//
+// A thread takes ZF consecutive fragments: most lie in one span, whose edge
+// values it steps from pixel to pixel as the reference does.
+
+// What bounds it: with many tiles, the latency of a tile's chain of loads (the
+// tile's spans, their triangles' records, the shading inputs), some 2.5 us a
+// step under load, which the few workgroups whose tiles fit a CU's LDS hide
+// less well than k_shade's and k_rop's many waves do; with heavy overdraw, the
+// depth recurrence.  Measured against k_frag_scan + k_shade + k_rop: textured
+// soup at 1080p 0.80 against 1.85 ms, a sphere and a cube at 512x512 21
+// against 56 us, a cube at 64x64 12 against 35, the 871,306-triangle mesh at
+// 1080p 54 against 61; but the same mesh at 7680x4320 0.54 against 0.48 ms
+// and its 4096x4096 depth map 0.20 against 0.15, where each pixel has half a
+// fragment.  So draws of at most ZTILES_DIRECT tiles take it as they are, and
+// of larger ones those with two fragments a pixel or more, which k_frag_scan
+// finds out on the device (DrawArgs::zpick).
+//
+// Sizes: the tile's depths, owners and colors (16 B a pixel) fill the LDS of
+// a CU with few workgroups, so a larger tile gets more threads; a draw of at
+// most ZTILES_FEW tiles leaves CUs idle and takes twice the threads a tile,
+// with shorter round sets (sphere and cube 33 -> 21 us).
+template <int ZT>
+struct ZSize {
+    static constexpr int B = ZT >= 1024 ? 128 : (ZT == 512 && TILE_PIX <= 2048 ? 512 : 256);  // spans staged at a time
+    static constexpr int CHUNK = ZT == 512 && TILE_PIX < 2048 ? 512 : 1024;                   // fragments of a round set
+    static constexpr int F = CHUNK / ZT;                                                     // of them a thread's
+    static constexpr int Q = ZT + CHUNK;  // queue entries: below a workgroup's worth before a round set
+    static_assert(B <= ZT && B % 64 == 0 && TILE_PIX <= 0x8000, "one staged span a thread; a pixel and a bit in 16");
+};
+constexpr int ZT_MANY = TILE_PIX >= 8192 ? 1024 : (TILE_PIX >= 2048 ? 512 : 256);
+constexpr int ZT_FEW = TILE_PIX >= 2048 ? ZT_MANY : 512;
+constexpr int ZTILES_FEW = 512;
+// The color of the fragment of span `si` at tile pixel `pix`
+// (context.go:208-238 from the span's first pixel on, then the shader).
+template <int SH, class G>
+FGL_D C4 shade_at(const G &g, uint32_t si, uint32_t pix) {
+    const DrawArgs &ka = g.args();
+    if (SH == 1) return c4(ka.sh.color[0], ka.sh.color[1], ka.sh.color[2], ka.sh.color[3]);
+    const Span sp = ka.spans[si];
+    TriIn t;
+    tri_from_rec(prim_of(ka, sp.ref), t);
+    ShadeIn in;
+    load_in<SH, false>(ka.sh, attr_src(ka), t.attr, in);
+    double w0 = sp.w[0], w1 = sp.w[1], w2 = sp.w[2];
+    const uint32_t j = pix - (uint32_t)sp.pix;
+#pragma unroll 4
+    for (uint32_t k = 0; k < j; k++) {
+        w0 += t.a12;
+        w1 += t.a20;
+        w2 += t.a01;
+    }
+    const double b0 = w0 * t.ra, b1 = w1 * t.ra, b2 = w2 * t.ra;
+    V4 bw = v4(b0 * t.r[0], b1 * t.r[1], b2 * t.r[2], 0);
+    bw.w = 1.0 / (bw.x + bw.y + bw.z);
+    return eval<SH>(ka.sh, in, bw);
+}
+
+// SH: 0 no color is written, 1 .. 4 as in k_shade.
+template <int SH, bool BLEND, int ZT, class G>
+FGL_D void zshade_body(const DrawArgs &a, const G &g) {
+    constexpr int ZB = ZSize<ZT>::B, ZCHUNK = ZSize<ZT>::CHUNK, ZF = ZSize<ZT>::F, ZQ = ZSize<ZT>::Q;
+    __shared__ double dep[TILE_PIX];
+    __shared__ uint32_t owner[TILE_PIX];
+    // opaque: the pixel's last survivor (span); blending: the pixel's color
+    __shared__ uint32_t out[SH == 0 ? 1 : TILE_PIX];
+    __shared__ __align__(16) Span zs[ZB];
+    __shared__ uint32_t excl[ZB + 1];
+    __shared__ uint32_t qspan[BLEND ? ZQ : 1];
+    __shared__ uint16_t qpix[BLEND ? ZQ : 1];
+    __shared__ uint32_t wsum[ZT / 64];
+    __shared__ uint64_t all;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int WAVES = ZT / 64;
+    __shared__ uint32_t again[3];  // some fragment of a round is still pending (in turn, zeroed a round ahead)
+    if (a.zpick && !a.ctr->zfirst) return;  // k_shade and k_rop draw it
+    const int t = (int)g.bid();
+    const uint32_t overflow = a.ctr->overflow, s0 = a.tstart[t], s1 = a.tend[t];
+    // every workgroup adds up the draw's fragments (TotalPixels: every
+    // fragment is an inside pixel with a valid index) and stops where they
+    // pass the capacity
+    if (tid < 3) again[tid] = 0;
+    if (wave == 0) {
+        uint64_t v = a.ctr->ftot[lane];
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+        if (lane == 0) all = v;
+    }
+    if (overflow) return;  // the host reruns the whole draw
+    __syncthreads();
+    const uint64_t total = all;
+    if (t == 0 && tid == 0) {
+        if (total > a.frag_lim) atomicOr(&a.ctr->overflow, 32u);
+        a.ctr->nfrags = total > a.frag_lim ? a.frag_lim : (uint32_t)total;
+        a.ctr->frags_lo = (uint32_t)total;
+        a.ctr->frags_hi = (uint32_t)(total >> 32);
+        a.ctr->total = total;
+    }
+    if (total > a.frag_lim) return;
+
+    const int tx = t % a.ntx, ty = t / a.ntx;
+    const int cx0 = tx * TILE_W, cy0 = ty * TILE_H;
+    const int cw = min(TILE_W, a.W - cx0), chh = min(TILE_H, a.H - cy0);
+    // the tile's blocks of deferred clears, as in k_rop
+    constexpr int TBW = TILE_W / CB_W, TBH = TILE_H / CB_H;
+    const int bx0 = cx0 / CB_W, by0 = cy0 / CB_H;
+    const int nbx = (cw + CB_W - 1) / CB_W, nby = (chh + CB_H - 1) / CB_H;
+    const bool my_block = tid < TBW * TBH && tid % TBW < nbx && tid / TBW < nby;
+    uint8_t *const my_mark = a.cblk + (by0 + tid / TBW) * a.cbw + bx0 + tid % TBW;
+    auto mark_of = [&](int lx, int ly) { return a.cblk[(by0 + ly / CB_H) * a.cbw + bx0 + lx / CB_W]; };
+
+    const double bias = a.st.depth_bias;
+    const bool rd = a.st.read_depth != 0, wd = a.st.write_depth != 0;
+    uint32_t my_updated = 0;
+    bool live = false;              // the tile's depth (and color) are in LDS
+    uint32_t qn = 0, qhead = 0;     // queued survivors
+
+    // ends a round: whether any thread's fragment is still pending (mine)
+    uint32_t round = 0;
+    auto more_rounds = [&](bool mine) {
+        const uint32_t next = round == 2 ? 0 : round + 1;
+        if (mine) again[round] = 1;
+        if (tid == 0) again[next] = 0;
+        __syncthreads();
+        const bool more = again[round] != 0;
+        round = next;
+        return more;
+    };
+
+    // shades the first n queued survivors and blends them in order
+    auto flush = [&](uint32_t n) {
+        uint32_t color = 0, pix = 0;
+        bool pend = (uint32_t)tid < n, over = false, inb = false;
+        if (pend) {
+            uint32_t at = qhead + (uint32_t)tid;
+            if (at >= (uint32_t)ZQ) at -= (uint32_t)ZQ;
+            pix = qpix[at] & 0x7fffu;
+            inb = (qpix[at] >> 15) != 0;
+            const C4 c = shade_at<SH == 0 ? 1 : SH>(g, qspan[at], pix);
+            color = nrgba_pack(c);
+            over = c.a < 1;
+        }
+        while (true) {
+            if (pend) atomicMin(&owner[pix], (uint32_t)tid);
+            __syncthreads();
+            if (pend && owner[pix] == (uint32_t)tid) {
+                if (over) out[pix] = blend_over(out[pix], color);
+                else if (inb) out[pix] = color;
+                pend = false;
+                owner[pix] = OWNER_NONE;
+            }
+            if (!more_rounds(pend)) break;
+        }
+        qhead += n;
+        if (qhead >= (uint32_t)ZQ) qhead -= (uint32_t)ZQ;
+        qn -= n;
+    };
+
+    for (uint32_t sb = s0; sb < s1; sb += ZB) {
+        // the next ZB spans and the positions of their fragments
+        uint32_t n = 0;
+        if (tid < ZB && sb + (uint32_t)tid < s1) {
+            const uint4 *src = reinterpret_cast<const uint4 *>(a.spans + sb + tid);
+            const uint4 lo = src[0], hi = src[1];
+            reinterpret_cast<uint4 *>(&zs[tid])[0] = lo;
+            reinterpret_cast<uint4 *>(&zs[tid])[1] = hi;
+            n = (hi.w >> 16) & SPAN_N;
+        }
+        uint32_t incl = n;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t y = __shfl_up(incl, off);
+            if (lane >= off) incl += y;
+        }
+        if (lane == 63) wsum[wave] = incl;
+        __syncthreads();
+        uint32_t T = 0;
+#pragma unroll
+        for (int w = 0; w < ZB / 64; w++) {
+            if (w < wave) incl += wsum[w];
+            T += wsum[w];
+        }
+        if (tid < ZB) excl[tid] = incl - n;
+        if (tid == 0) excl[ZB] = T;
+        if (T != 0 && !live) {
+            // the tile's current depth (and, to blend into, color): the
+            // pending clear, a marked block's clear, or memory
+            live = true;
+            constexpr int PPT = TILE_PIX / ZT;
+            const bool all_pending = a.clear_depth_pending && (!BLEND || a.clear_color_pending);
+            uint8_t mk[PPT];
+#pragma unroll
+            for (int k = 0; k < PPT; k++) {
+                const int p = k * ZT + tid;
+                const int lx = p % TILE_W, ly = p / TILE_W;
+                mk[k] = lx < cw && ly < chh && !all_pending ? mark_of(lx, ly) : (uint8_t)0;
+            }
+#pragma unroll
+            for (int k = 0; k < PPT; k++) {
+                const int p = k * ZT + tid;
+                const int lx = p % TILE_W, ly = p / TILE_W;
+                const int64_t gi = (int64_t)(cy0 + (ly < chh ? ly : 0)) * a.W + cx0 + (lx < cw ? lx : 0);
+                double dv = a.clear_depth;
+                if (!a.clear_depth_pending && !(mk[k] & CB_DEPTH)) dv = a.depth[gi];
+                dep[p] = dv;
+                owner[p] = OWNER_NONE;
+                if (SH != 0) {
+                    uint32_t cv = OWNER_NONE;
+                    if (BLEND) {
+                        cv = a.clear_color;
+                        if (!a.clear_color_pending && !(mk[k] & CB_COLOR)) cv = a.color[gi];
+                    }
+                    out[p] = cv;
+                }
+            }
+        }
+        __syncthreads();
+        for (uint32_t c0 = 0; c0 < T; c0 += ZCHUNK) {
+            double z[ZF];
+            uint32_t px[ZF];  // staged span << 16 | in bounds << 15 | pixel
+            uint32_t pending = 0;
+            const uint32_t p0 = c0 + (uint32_t)(ZF * tid);
+            if (p0 < T) {
+                // the span of the first fragment: the last one starting at
+                // or before it
+                uint32_t o = 0;
+#pragma unroll
+                for (int st = ZB / 2; st > 0; st >>= 1)
+                    if (excl[o + st] <= p0) o += st;
+                double w0 = 0, w1 = 0, w2 = 0, a12 = 0, a20 = 0, a01 = 0, ra = 0, z0 = 0, z1 = 0, z2 = 0;
+                uint32_t pn = 0, start = 0, end = 0;
+#pragma unroll
+                for (int q = 0; q < ZF; q++) {
+                    const uint32_t p = p0 + (uint32_t)q;
+                    z[q] = 0;
+                    px[q] = 0;
+                    if (p < T) {
+                        if (q == 0 || p >= end) {
+                            if (q > 0)
+                                do o++;
+                                while (excl[o + 1] <= p);
+                            const Span s = zs[o];
+                            const PrimRec *pr = prim_of(a, s.ref);
+                            const double y0 = pr->sy[0], y1 = pr->sy[1], y2 = pr->sy[2];
+                            z0 = pr->sz[0];
+                            z1 = pr->sz[1];
+                            z2 = pr->sz[2];
+                            ra = pr->ra;
+                            a12 = y2 - y1;
+                            a20 = y0 - y2;
+                            a01 = y1 - y0;
+                            w0 = s.w[0];
+                            w1 = s.w[1];
+                            w2 = s.w[2];
+                            pn = (uint32_t)s.pix | ((uint32_t)(s.n & SPAN_INB));
+                            start = excl[o];
+                            end = excl[o + 1];
+                            // the reference's per-pixel step up to the first fragment (context.go:208-213)
+                            if (q == 0)
+                                for (uint32_t k = start; k < p; k++) {
+                                    w0 += a12;
+                                    w1 += a20;
+                                    w2 += a01;
+                                }
+                        } else {
+                            w0 += a12;
+                            w1 += a20;
+                            w2 += a01;
+                        }
+                        const double b0 = w0 * ra, b1 = w1 * ra, b2 = w2 * ra;
+                        z[q] = b0 * z0 + b1 * z1 + b2 * z2;  // context.go:230
+                        px[q] = (o << 16) | (pn + (p - start));
+                        pending |= 1u << q;
+                    }
+                }
+            }
+            uint32_t passed = 0;
+            while (true) {
+#pragma unroll
+                for (int q = 0; q < ZF; q++)
+                    if (pending & (1u << q)) atomicMin(&owner[px[q] & 0x7fffu], (uint32_t)(ZF * tid + q));
+                __syncthreads();
+#pragma unroll
+                for (int q = 0; q < ZF; q++) {
+                    if (!(pending & (1u << q))) continue;
+                    const uint32_t p = px[q] & 0x7fffu;
+                    if (owner[p] != (uint32_t)(ZF * tid + q)) continue;
+                    // context.go:230-273 at this pixel, in order
+                    const double bz = z[q] + bias;
+                    if (!(rd && bz > dep[p]) && (bz <= dep[p] || !rd)) {
+                        my_updated++;
+                        if (wd) dep[p] = z[q];
+                        if (BLEND) passed |= 1u << q;
+                        else if (SH != 0 && (px[q] & 0x8000u)) out[p] = sb + (px[q] >> 16);
+                    }
+                    pending &= ~(1u << q);
+                    owner[p] = OWNER_NONE;
+                }
+                if (!more_rounds(pending != 0)) break;
+            }
+            if (BLEND) {
+                // the survivors, in order, behind those queued
+                const uint32_t mine = (uint32_t)__popc(passed);
+                uint32_t v = mine;
+                for (int off = 1; off < 64; off <<= 1) {
+                    const uint32_t y = __shfl_up(v, off);
+                    if (lane >= off) v += y;
+                }
+                if (lane == 63) wsum[wave] = v;
+                __syncthreads();
+                uint32_t at = qn + v - mine, more = 0;
+#pragma unroll
+                for (int w = 0; w < WAVES; w++) {
+                    const uint32_t x = wsum[w];
+                    if (w < wave) at += x;
+                    more += x;
+                }
+                at += qhead;
+                if (at >= (uint32_t)ZQ) at -= (uint32_t)ZQ;
+#pragma unroll
+                for (int q = 0; q < ZF; q++)
+                    if (passed & (1u << q)) {
+                        qspan[at] = sb + (px[q] >> 16);
+                        qpix[at] = (uint16_t)px[q];
+                        if (++at == (uint32_t)ZQ) at = 0;
+                    }
+                qn += more;
+                __syncthreads();
+                while (qn >= (uint32_t)ZT) flush(ZT);
+            }
+        }
+    }
+    if (!live) {
+        // no fragment: a pending clear stays deferred, marked on the blocks
+        const uint8_t bits = (a.clear_color_pending ? CB_COLOR : 0) | (a.clear_depth_pending ? CB_DEPTH : 0);
+        if (bits && my_block) *my_mark |= bits;
+        return;
+    }
+    if (BLEND && qn) flush(qn);
+
+    for (int p = tid; p < TILE_PIX; p += ZT) {
+        const int lx = p % TILE_W, ly = p / TILE_W;
+        if (lx < cw && ly < chh) {
+            const int64_t gi = (int64_t)(cy0 + ly) * a.W + cx0 + lx;
+            a.depth[gi] = dep[p];
+            if (BLEND) a.color[gi] = out[p];
+        }
+    }
+    if (SH != 0 && !BLEND) {
+        // 8 x 8 pixels a wave: the pixels of few triangles
+        constexpr int BW = TILE_W / 8, NB = TILE_PIX / 64;
+        for (int b = wave; b < NB; b += WAVES) {
+            const int lx = (b % BW) * 8 + (lane & 7), ly = (b / BW) * 8 + (lane >> 3);
+            if (lx >= cw || ly >= chh) continue;
+            const int p = ly * TILE_W + lx;
+            const int64_t gi = (int64_t)(cy0 + ly) * a.W + cx0 + lx;
+            const uint32_t si = out[p];
+            if (si != OWNER_NONE) a.color[gi] = nrgba_pack(shade_at<SH == 0 ? 1 : SH>(g, si, (uint32_t)p));
+            else if (a.clear_color_pending || (mark_of(lx, ly) & CB_COLOR)) a.color[gi] = a.clear_color;
+        }
+    }
+    __syncthreads();  // every thread has read its marks
+    // the whole tile is written: its blocks hold no deferred clear, but a
+    // color nothing wrote keeps its own
+    if (my_block)
+        *my_mark = SH == 0 && (a.clear_color_pending || (*my_mark & CB_COLOR)) ? CB_COLOR : (uint8_t)0;
+    // UpdatedPixels of this tile, into one of the partial sums
+    for (int off = 32; off > 0; off >>= 1) my_updated += __shfl_down(my_updated, off);
+    if (lane == 0) wsum[wave] = my_updated;
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t s = 0;
+        for (int w = 0; w < WAVES; w++) s += wsum[w];
+        if (s) atomicAdd(&a.ctr->upd[t % UPD_PARTS], s);
+    }
+}
+template <int SH, bool BLEND, int ZT>
+__global__ __launch_bounds__(ZT, 4) void k_zshade(DrawArgs a) {
+    zshade_body<SH, BLEND, ZT>(a, OneDraw{});
+}
+template <int SH, bool BLEND>
+__global__ __launch_bounds__(ZT_MANY, 4) void k_zshade_m(MultiArgs m) {
+    const ManyDraws g = many_draws(m);
+    zshade_body<SH, BLEND, ZT_MANY>(draw_of(g), g);
+}
+
+// The variant of a draw's k_zshade: 0 .. 4 opaque by SH, 5 .. 8 blending.
+static int zshade_variant(const DrawArgs &a) {
+    if (!a.st.write_color) return 0;
+    const int sh = a.sh.kind == 3 && a.sh.has_tex ? 4 : a.sh.kind;
+    return a.zmode == 2 ? 4 + sh : sh;
+}
+#define FGL_ZSHADE_CASES(LAUNCH)            \
+    switch (zshade_variant(rep)) {          \
+        case 0: LAUNCH(0, false); break;    \
+        case 1: LAUNCH(1, false); break;    \
+        case 2: LAUNCH(2, false); break;    \
+        case 3: LAUNCH(3, false); break;    \
+        case 4: LAUNCH(4, false); break;    \
+        case 5: LAUNCH(1, true); break;     \
+        case 6: LAUNCH(2, true); break;     \
+        case 7: LAUNCH(3, true); break;     \
+        default: LAUNCH(4, true); break;    \
+    }
+hipError_t launch_zshade(const DrawArgs &rep, hipStream_t s) {
+    const dim3 grid(rep.ntiles);
+    if (rep.ntiles <= ZTILES_FEW) {
+#define FGL_LAUNCH(SH, BL) hipLaunchKernelGGL((k_zshade<SH, BL, ZT_FEW>), grid, dim3(ZT_FEW), 0, s, rep)
+        FGL_ZSHADE_CASES(FGL_LAUNCH)
+#undef FGL_LAUNCH
+    } else {
+#define FGL_LAUNCH(SH, BL) hipLaunchKernelGGL((k_zshade<SH, BL, ZT_MANY>), grid, dim3(ZT_MANY), 0, s, rep)
+        FGL_ZSHADE_CASES(FGL_LAUNCH)
+#undef FGL_LAUNCH
+    }
+    return hipGetLastError();
+}
+static hipError_t launch_zshade_multi(const MultiArgs &m, uint32_t nb, const DrawArgs &rep, hipStream_t s) {
+#define FGL_LAUNCH(SH, BL) hipLaunchKernelGGL((k_zshade_m<SH, BL>), dim3(nb), dim3(ZT_MANY), 0, s, m)
+    FGL_ZSHADE_CASES(FGL_LAUNCH)
+#undef FGL_LAUNCH
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 
 static unsigned span_grid(const DrawArgs &a) {
     const uint64_t nb = ((uint64_t)a.span_cap + SPAN_THREADS - 1) / SPAN_THREADS;  // workgroups of 4 waves
@@ -904,6 +1347,7 @@ uint32_t stage_blocks(int stage, const DrawArgs &a, bool many) {
         case ST_FRAG_SCAN: return frag_groups(a);
         case ST_SHADE: return span_grid(a);
         case ST_ROP: return (uint32_t)a.ntiles;
+        case ST_ZSHADE: return (uint32_t)a.ntiles;
         default: return 0;
     }
 }
@@ -913,7 +1357,7 @@ hipError_t launch_multi(int stage, const MultiArgs &m, uint32_t nblocks, const D
         launch_zero_multi,       launch_vs_multi,         launch_vs_deferred_multi, launch_scan_top_multi,
         launch_emit_multi,       launch_radix_hist_multi, launch_radix_scan_multi,  launch_radix_scatter_multi,
         launch_span_count_multi, launch_span_scan_multi,  launch_spans_multi,       launch_frag_scan_multi,
-        launch_shade_multi,      launch_rop_multi,
+        launch_shade_multi,      launch_rop_multi,        launch_zshade_multi,
     };
     if (stage < 0 || stage >= ST_COUNT) return hipErrorInvalidValue;
     if (nblocks == 0) return hipSuccess;
@@ -944,6 +1388,7 @@ const TileOps &FGL_OPS1(FGL_TILE_W, FGL_TILE_H)() {
         FGL_TILE_NS::launch_frag_scan,
         FGL_TILE_NS::launch_shade,
         FGL_TILE_NS::launch_tile,
+        FGL_TILE_NS::launch_zshade,
         FGL_TILE_NS::stage_blocks,
         FGL_TILE_NS::launch_multi,
     };
