@@ -675,7 +675,7 @@ def LoadSTL(ctx, src):
     """LoadSTL (stl.go:23-57) into a mesh resident on ctx's device; src is a
     path or the file's bytes."""
     data = _file_bytes(src)
-    buf = (ctypes.c_uint8 * max(len(data), 1)).from_buffer_copy(data or b"\0")
+    buf = ctypes.cast(ctypes.c_char_p(data), ctypes.POINTER(ctypes.c_uint8))
     h = ctypes.c_void_p()
     N.check(N.load().fgl_mesh_load_stl(ctx._ptr(), buf, len(data), ctypes.byref(h)), ctx._ptr())
     return DeviceMesh(ctx, None, handle=h)
