@@ -871,7 +871,12 @@ FGL_DRAW_KERNELS(k_rop, rop_body, __launch_bounds__(TILE_THREADS, FGL_ROP_WAVES)
 // and its 4096x4096 depth map 0.20 against 0.15, where each pixel has half a
 // fragment.  So draws of at most ZTILES_DIRECT tiles take it as they are, and
 // of larger ones those with two fragments a pixel or more, which k_frag_scan
-// finds out on the device (DrawArgs::zpick).
+// finds out on the device (DrawArgs::zpick).  The device also picks for draws
+// of more than ZTILE_DENSE primitives a tile, whose spans of a pixel or two
+// leave each fragment a load of its own: whole draws at 1024x1024 of 871,306
+// triangles 311 us tested first, 289 picked; of 400,000 231 and 228; but of
+// 155,000 213 and 215, of 20,000 157 and 158.  With at most ZTILES_FEW tiles
+// the two differ by less than 4 us at any density.
 //
 // Sizes: the tile's depths, owners and colors (16 B a pixel) fill the LDS of
 // a CU with few workgroups, so a larger tile gets more threads; a draw of at
@@ -887,7 +892,6 @@ struct ZSize {
 };
 constexpr int ZT_MANY = TILE_PIX >= 8192 ? 1024 : (TILE_PIX >= 2048 ? 512 : 256);
 constexpr int ZT_FEW = TILE_PIX >= 2048 ? ZT_MANY : 512;
-constexpr int ZTILES_FEW = 512;
 // The color of the fragment of span `si` at tile pixel `pix`
 // (context.go:208-238 from the span's first pixel on, then the shader).
 template <int SH, class G>

@@ -122,3 +122,14 @@ def test_many_tiles(shader, size, deep):
     prims = _soup(60, 4, 0.9) if deep else _soup(40, 5, 0.1)
     ctx = _check(f"{shader}, {W}x{H}, deep {deep}", SHADERS[shader](), W, H, [prims], [{}])
     assert (ctx.DrawStats()["fragments"] >= 2 * W * H) == deep
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [102400, 102401])
+@pytest.mark.parametrize("deep", [True, False])
+def test_dense_triangles(n, deep):
+    # 800 tiles: at 128 triangles a tile depth first, above it the device picks
+    W, H = 1000, 800
+    prims = _soup(n, 6, 0.03 if deep else 0.004)
+    ctx = _check(f"{n} triangles, deep {deep}", SHADERS["phong"](), W, H, [prims], [{}])
+    assert (ctx.DrawStats()["fragments"] >= 2 * W * H) == deep
