@@ -1,9 +1,9 @@
 """Readbacks through the page-locked chunks and buffers made from blocks that
 earlier objects let go.
 
-A readback is cut into chunks of a quarter of its size, at least 512 KiB and
-at most 1 MiB, in a ring of four: the sizes below lie on both sides of one
-chunk, of several, and of the ring's wrap-around.  Bytes come back unchanged,
+A readback above 768 KiB is cut into chunks of a quarter of its size, at
+least 512 KiB and at most 1 MiB, in a ring of four: the sizes below lie on both
+sides of one chunk, of several, and of the ring's wrap-around.  Bytes come back unchanged,
 so every comparison is exact."""
 import threading
 
@@ -24,7 +24,7 @@ def _pattern(w, h, seed):
     return np.random.default_rng(seed).integers(0, 256, (h, w, 4), dtype=np.uint8)
 
 
-@pytest.mark.parametrize("w,h", [(1, 1), (131072, 1), (131073, 1), (131071, 1), (512, 512), (1023, 769),
+@pytest.mark.parametrize("w,h", [(1, 1), (131072, 1), (131073, 1), (131071, 1), (512, 384), (513, 384), (512, 512), (1023, 769),
                                  (1024, 1024), (1025, 1024), (2049, 512), (3000, 1777)])
 def test_image_round_trip(w, h):
     _say(f"image {w}x{h}")
