@@ -826,8 +826,9 @@ int draw_begin(fgl_ctx *c, const fgl_state *st, const fgl_shader *sh, int kind, 
     }
     T = draw_ops(c, kind, in.n);
     draw_setup(c, st, *T, kind, in, a);
-    a.zmode = draw_zmode(a);
-    a.zpick = a.zmode && (a.ntiles > ZTILES_DIRECT || (a.ntiles > ZTILES_FEW && in.n > (int64_t)ZTILE_DENSE * a.ntiles));
+    a.zmode = T->tw * T->th <= ZTILE_PIX ? draw_zmode(a) : 0;
+    a.zpick = a.zmode && (a.ntiles > ZTILES_DIRECT ||
+                          ((int64_t)a.W * a.H > ZDENSE_PIX && in.n > (int64_t)ZTILE_DENSE * a.ntiles));
     const int64_t n = in.n;
 
     // starting capacities; grown on overflow

@@ -98,10 +98,11 @@ constexpr int VS_THREADS = 256;
 // Tiles up to which a draw that can be tested first is (see k_zshade): a
 // 1080p frame's, about two rounds of resident workgroups.
 constexpr int ZTILES_DIRECT = 2304;
-// Tiles up to which k_zshade takes twice the threads a tile, and primitives a
-// tile above which a draw of more tiles leaves the choice to the device.
-constexpr int ZTILES_FEW = 512;
+// Primitives a tile above which a frame of more than ZDENSE_PIX pixels leaves
+// the choice to the device, and the largest tile that is tested first.
 constexpr int ZTILE_DENSE = 128;
+constexpr int64_t ZDENSE_PIX = 512 * 1024;
+constexpr int ZTILE_PIX = 2048;
 constexpr int SPAN_THREADS = 256;
 constexpr int SPAN_GROUP = 64;  // pairs whose spans are placed together
 // Spans per fragment-count block: the shading kernel's waves each take one

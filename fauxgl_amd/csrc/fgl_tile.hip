@@ -875,8 +875,11 @@ FGL_DRAW_KERNELS(k_rop, rop_body, __launch_bounds__(TILE_THREADS, FGL_ROP_WAVES)
 // of more than ZTILE_DENSE primitives a tile, whose spans of a pixel or two
 // leave each fragment a load of its own: whole draws at 1024x1024 of 871,306
 // triangles 311 us tested first, 289 picked; of 400,000 231 and 228; but of
-// 155,000 213 and 215, of 20,000 157 and 158.  With at most ZTILES_FEW tiles
-// the two differ by less than 4 us at any density.
+// 155,000 213 and 215, of 20,000 157 and 158.  In frames of at most ZDENSE_PIX
+// pixels the two differ by less than 4 us at any density.  Tiles of more than
+// ZTILE_PIX pixels leave one workgroup a CU, and too few at that: the 871,306
+// triangles at 1080p 198 us in 128x64 tiles and 109 in 64x64, against 61; a
+// sphere and a cube 110 and 67.  They are shaded first.
 //
 // Sizes: the tile's depths, owners and colors (16 B a pixel) fill the LDS of
 // a CU with few workgroups, so a larger tile gets more threads; a draw of at
@@ -884,14 +887,15 @@ FGL_DRAW_KERNELS(k_rop, rop_body, __launch_bounds__(TILE_THREADS, FGL_ROP_WAVES)
 // with shorter round sets (sphere and cube 33 -> 21 us).
 template <int ZT>
 struct ZSize {
-    static constexpr int B = ZT >= 1024 ? 128 : (ZT == 512 && TILE_PIX <= 2048 ? 512 : 256);  // spans staged at a time
-    static constexpr int CHUNK = ZT == 512 && TILE_PIX < 2048 ? 512 : 1024;                   // fragments of a round set
-    static constexpr int F = CHUNK / ZT;                                                     // of them a thread's
+    static constexpr int B = ZT;                                                 // spans staged at a time
+    static constexpr int CHUNK = ZT == 512 && TILE_PIX < 2048 ? 512 : 1024;      // fragments of a round set
+    static constexpr int F = CHUNK / ZT;                                         // of them a thread's
     static constexpr int Q = ZT + CHUNK;  // queue entries: below a workgroup's worth before a round set
     static_assert(B <= ZT && B % 64 == 0 && TILE_PIX <= 0x8000, "one staged span a thread; a pixel and a bit in 16");
 };
-constexpr int ZT_MANY = TILE_PIX >= 8192 ? 1024 : (TILE_PIX >= 2048 ? 512 : 256);
-constexpr int ZT_FEW = TILE_PIX >= 2048 ? ZT_MANY : 512;
+constexpr int ZT_MANY = TILE_PIX >= 2048 ? 512 : 256;
+constexpr int ZT_FEW = 512;
+constexpr int ZTILES_FEW = 512;
 // The color of the fragment of span `si` at tile pixel `pix`
 // (context.go:208-238 from the span's first pixel on, then the shader).
 template <int SH, class G>
@@ -1243,6 +1247,7 @@ __global__ __launch_bounds__(ZT_MANY, 4) void k_zshade_m(MultiArgs m) {
     zshade_body<SH, BLEND, ZT_MANY>(draw_of(g), g);
 }
 
+#if FGL_TILE_W * FGL_TILE_H <= 2048  // ZTILE_PIX
 // The variant of a draw's k_zshade: 0 .. 4 opaque by SH, 5 .. 8 blending.
 static int zshade_variant(const DrawArgs &a) {
     if (!a.st.write_color) return 0;
@@ -1280,6 +1285,12 @@ static hipError_t launch_zshade_multi(const MultiArgs &m, uint32_t nb, const Dra
 #undef FGL_LAUNCH
     return hipGetLastError();
 }
+#else  // never asked for
+hipError_t launch_zshade(const DrawArgs &, hipStream_t) { return hipErrorInvalidValue; }
+static hipError_t launch_zshade_multi(const MultiArgs &, uint32_t, const DrawArgs &, hipStream_t) {
+    return hipErrorInvalidValue;
+}
+#endif
 
 // ---------------------------------------------------------------------------
 
