@@ -126,6 +126,10 @@ struct DrawCounters {
     unsigned long long ftot[64];
 };
 constexpr int UPD_PARTS = 64;
+// DrawCounters::overflow: fragments past the capacity.  The kernels that find
+// it (k_shade, k_zshade) set it themselves; every other bit is set by a kernel
+// before them.
+constexpr uint32_t OVF_FRAGS = 32u;
 
 // Coverage span: the covered pixels of one row of one raster triangle in
 // one tile, with the edge values the reference holds at the first of them.

@@ -543,7 +543,10 @@ FGL_D void shade_body(const DrawArgs &a, const G &grid) {
     __shared__ double slots[SPAN_THREADS / 64][SHADE_SLOTS][L::N];
     __shared__ uint64_t gpre[FRAG_GTAB];  // exclusive prefix of the group sums
     __shared__ uint64_t gw[SPAN_THREADS / 64];
-    if (a.ctr->overflow || a.ctr->zfirst) return;
+    // Not the fragments' own bit: workgroup 0 may set it in this launch, and
+    // the waves of a workgroup that read it before and after would part at the
+    // barriers below.  Every workgroup compares the total itself.
+    if ((a.ctr->overflow & ~OVF_FRAGS) || a.ctr->zfirst) return;
     const uint32_t NS = a.ctr->nspans;
     const uint32_t nb = (NS + FRAG_BLOCK - 1) / FRAG_BLOCK;
     const uint32_t ngroups = (nb + FRAG_GROUP - 1) / FRAG_GROUP;
@@ -571,7 +574,7 @@ FGL_D void shade_body(const DrawArgs &a, const G &grid) {
         __syncthreads();
     }
     if (grid.bid() == 0 && threadIdx.x == 0) {
-        if (total > a.frag_cap) atomicOr(&a.ctr->overflow, 32u);
+        if (total > a.frag_cap) atomicOr(&a.ctr->overflow, OVF_FRAGS);
         a.ctr->nfrags = total > a.frag_cap ? a.frag_cap : (uint32_t)total;
         a.ctr->frags_lo = (uint32_t)total;
         a.ctr->frags_hi = (uint32_t)(total >> 32);
@@ -940,7 +943,8 @@ FGL_D void zshade_body(const DrawArgs &a, const G &g) {
     __shared__ uint32_t again[3];  // some fragment of a round is still pending (in turn, zeroed a round ahead)
     if (a.zpick && !a.ctr->zfirst) return;  // k_shade and k_rop draw it
     const int t = (int)g.bid();
-    const uint32_t overflow = a.ctr->overflow, s0 = a.tstart[t], s1 = a.tend[t];
+    // (not the fragments' bit, which this launch may set: as in k_shade)
+    const uint32_t overflow = a.ctr->overflow & ~OVF_FRAGS, s0 = a.tstart[t], s1 = a.tend[t];
     // every workgroup adds up the draw's fragments (TotalPixels: every
     // fragment is an inside pixel with a valid index) and stops where they
     // pass the capacity
@@ -954,7 +958,7 @@ FGL_D void zshade_body(const DrawArgs &a, const G &g) {
     __syncthreads();
     const uint64_t total = all;
     if (t == 0 && tid == 0) {
-        if (total > a.frag_lim) atomicOr(&a.ctr->overflow, 32u);
+        if (total > a.frag_lim) atomicOr(&a.ctr->overflow, OVF_FRAGS);
         a.ctr->nfrags = total > a.frag_lim ? a.frag_lim : (uint32_t)total;
         a.ctr->frags_lo = (uint32_t)total;
         a.ctr->frags_hi = (uint32_t)(total >> 32);

@@ -133,3 +133,40 @@ def test_dense_triangles(n, deep):
     prims = _soup(n, 6, 0.03 if deep else 0.004)
     ctx = _check(f"{n} triangles, deep {deep}", SHADERS["phong"](), W, H, [prims], [{}])
     assert (ctx.DrawStats()["fragments"] >= 2 * W * H) == deep
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shader", ["solid translucent", "texture", "phong", "texture with a hole"])
+@pytest.mark.parametrize("size,n", [((97, 67), 60), ((1000, 800), 300), ((1600, 1504), 300)])
+def test_forced_fragment_overflow(shader, size, n):
+    """A draw over opaque pixels whose first pass runs out of fragments: no
+    tile of that pass may draw, whichever of its workgroups sees the overflow
+    set by another first; blended pixels drawn twice would differ.  800 and 2350
+    tiles are more than are resident at once; the draw with a hole is shaded first."""
+    W, H = size
+    _say(f"depth first: forced fragment overflow, {shader}, {W}x{H}")
+    below, prims = _soup(40, 8, 0.9), _soup(n, 9, 0.7)
+    octx, ctx = O.Context(W, H), A.NewContext(W, H)
+    ctx.Cull = A.CullNone
+    octx.set_state(O.make_state(front_face=O.FACE_CCW, line_width=2.0, read_depth=True, write_depth=True,
+                                write_color=True, alpha_blend=True, wireframe=False, cull=A.CullNone, depth_bias=0.0))
+    ctx.Shader = SHADERS[shader]()
+    ctx.DrawTriangles(prims)  # sizes the other buffers
+    for bg in (A.White, A.Color(0.1, 0.2, 0.3, 0.5)):
+        ri, gi = [], []
+        octx.clear_color(tuple(bg))
+        octx.clear_depth(A.MaxFloat64)
+        ctx.ClearColorBufferWith(bg)
+        ctx.ClearDepthBuffer()
+        for p, name, forced in ((below, "solid", False), (prims, shader, True)):
+            sh = SHADERS[name]()
+            octx.set_shader(oracle_shader(sh))
+            ctx.Shader = sh
+            ri.append(octx.draw_triangles(O.Mesh(tris=p.arrays()), 1))
+            if forced:
+                ctx.ForceCapacities(fragments=1)
+            gi.append(tuple(ctx.DrawTriangles(p)))
+        st = ctx.DrawStats()
+        assert st["overflow_mask"] == 32 and st["reruns"] == 1, st
+        res = compare((octx.color(), octx.depth(), ri), (ctx.Image(), ctx.DepthBuffer, gi), color_tol=0)
+        assert res["ok"], res
