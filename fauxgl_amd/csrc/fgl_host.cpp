@@ -2961,14 +2961,40 @@ int batch_eager(fgl_batch *b, size_t i, uint64_t info[2]) {
     return FGL_OK;
 }
 
-// Records every view into one graph.  Nothing is allocated while recording
-// unless a capacity moved since the eager pass; then the addresses of the
-// views recorded earlier may be stale, and the recording is made again.
+// Sizes every buffer the views' draws use for their contexts' capacities.  The
+// eager pass does not: a later draw of the context may have raised a capacity
+// without using the buffers behind it (a draw that is tested first writes no
+// fragments).
+int batch_size_buffers(fgl_batch *b) {
+    for (size_t i = 0; i < b->views.size(); i++) {
+        fgl_batch::View &v = b->views[i];
+        for (int kind : {(int)PRIM_TRI, (int)PRIM_LINE}) {
+            DevPrims p;
+            mesh_prims(v.mesh, kind == PRIM_LINE, p);
+            if (p.n == 0) continue;
+            DrawArgs a;
+            const TileOps *T;
+            int r = draw_begin(v.ctx, &v.st, &v.sh, kind, p, T, a);
+            if (!r) r = draw_buffers(v.ctx, a);
+            if (r) {
+                set_err(b->err, "view %zu: %s", i, v.ctx->err.c_str());
+                return r;
+            }
+        }
+    }
+    return FGL_OK;
+}
+
+// Records every view into one graph.  A capture refuses allocations, frees
+// and waits, so the buffers are sized first; should one move all the same (a
+// tuning table loaded meanwhile), the recording fails or is made again.
 int batch_record(fgl_batch *b) {
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
     if (b->graph) (void)hipGraphDestroy(b->graph);
     b->exec = nullptr;
     b->graph = nullptr;
+    int r = batch_size_buffers(b);
+    if (r) return r;
     std::vector<fgl_ctx *> &ctxs = b->ctxs;
     while (b->joins.size() < ctxs.size()) {
         hipEvent_t e;
@@ -2982,7 +3008,6 @@ int batch_record(fgl_batch *b) {
     }
     const uint64_t epoch0 = g_dev_epoch.load();
     BCHK(b, hipStreamBeginCapture(b->s0, hipStreamCaptureModeThreadLocal));
-    int r = FGL_OK;
     if (hipEventRecord(b->fork, b->s0) != hipSuccess) r = FGL_E_DEVICE;
     for (size_t k = 0; k < ctxs.size() && !r; k++)
         if (hipStreamWaitEvent(ctxs[k]->stream, b->fork, 0) != hipSuccess) r = FGL_E_DEVICE;
