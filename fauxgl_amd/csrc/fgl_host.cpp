@@ -119,6 +119,7 @@ thread_local int g_idle_dev = -1;
 struct DeviceIdle {
     explicit DeviceIdle(int dev) {
         if (hipDeviceSynchronize() == hipSuccess) g_idle_dev = dev;
+        else (void)hipGetLastError();
     }
     ~DeviceIdle() { g_idle_dev = -1; }
 };
@@ -133,7 +134,10 @@ struct DevBuf {
         bool idle = g_idle_dev == dev;
         if (!idle && bytes <= kPoolBlock) {
             int cur = -1;
-            idle = hipGetDevice(&cur) == hipSuccess && cur == dev && hipDeviceSynchronize() == hipSuccess;
+            if (hipGetDevice(&cur) == hipSuccess && cur == dev) {
+                idle = hipDeviceSynchronize() == hipSuccess;
+                if (!idle) (void)hipGetLastError();  // refused (a capture is open): no error of a later call
+            }
         }
         if (idle && bytes <= kPoolBlock)
             pool_put(dev, p, bytes);
