@@ -956,5 +956,13 @@ def ClearTuning():
     N.check(N.load().fgl_tune_clear())
 
 
+def TrimMemory(device=-1):
+    """Gives back the device memory (of one device, or all) and the
+    page-locked memory that the library keeps for its next objects: at most 512
+    MiB and 16 MiB.  It does so by itself before an allocation of its own is
+    refused; this is for the process's other allocators."""
+    N.check(N.load().fgl_trim(device))
+
+
 def NewContext(width, height):
     return Context(width, height)

@@ -49,8 +49,9 @@ std::atomic<uint64_t> g_dev_epoch{0};
 // here only after the device has been idle since its buffer's last use (what
 // hipFree waits for as well), so whichever stream or thread takes it next
 // finds no work on it.  Blocks above kPoolBlock are freed at once; beyond
-// kPoolBytes or kPoolCount the oldest are; all are before an allocation is
-// refused.
+// kPoolBytes or kPoolCount the oldest are; all of a device's are before one
+// of the library's allocations there is refused, and all at fgl_trim (for the
+// process's other allocators).
 constexpr size_t kPoolBlock = (size_t)128 << 20, kPoolBytes = (size_t)512 << 20;
 constexpr int kPoolCount = 128;
 struct PoolBlock {
@@ -100,13 +101,14 @@ void pool_put(int dev, void *p, size_t bytes) {
     for (int k = 0; k < nd; k++) (void)hipFree(drop[k].p);
 }
 
+// frees what is kept of a device's blocks (-1: every device's)
 void pool_empty(int dev) {
     for (;;) {
         PoolBlock b{};
         {
             std::lock_guard<std::mutex> lk(g_pool_mu);
             for (int k = 0; k < g_pool_n && !b.p; k++)
-                if (g_pool[k].dev == dev) b = pool_take(k);
+                if (dev < 0 || g_pool[k].dev == dev) b = pool_take(k);
         }
         if (!b.p) return;
         (void)hipFree(b.p);
@@ -292,6 +294,19 @@ void stage_put(Stage *s) {
     delete s;
 }
 
+// frees the kept page-locked buffers
+void stages_empty() {
+    for (Stage *&kept : g_stages) {
+        Stage *s;
+        {
+            std::lock_guard<std::mutex> lk(g_stage_mu);
+            s = kept;
+            kept = nullptr;
+        }
+        delete s;
+    }
+}
+
 // memory the runtime knows (page-locked or device memory): copied as it is
 bool hip_knows(const void *p) {
     hipPointerAttribute_t at{};
@@ -344,7 +359,7 @@ hipError_t copy_out(int device, void *dst, const void *src, size_t n, hipStream_
 }
 
 struct Tex {
-    void *d = nullptr;
+    DevBuf d;
     int32_t w = 0, h = 0, kind = 0;
     bool solid = false;  // no texel of alpha 0
 };
@@ -413,11 +428,6 @@ struct fgl_ctx {
     std::vector<hipEvent_t> pool;
 
     ~fgl_ctx() {
-        for (auto &kv : tex)
-            if (kv.second.d) {
-                (void)hipFree(kv.second.d);
-                g_dev_epoch++;
-            }
         for (auto &p : pending) {
             (void)hipEventDestroy(p.a);
             (void)hipEventDestroy(p.b);
@@ -645,7 +655,7 @@ int fill_shader(fgl_ctx *c, const fgl_shader *sh, DevShader &d) {
         d.tex_kind = it->second.kind;
         d.tex_w = it->second.w;
         d.tex_h = it->second.h;
-        d.tex_pix = it->second.d;
+        d.tex_pix = it->second.d.p;
         d.tex_solid = it->second.solid;
     }
     return FGL_OK;
@@ -1081,6 +1091,13 @@ int fgl_init(int32_t device) {
 
 const char *fgl_last_error(const fgl_ctx *ctx) { return ctx ? ctx->err.c_str() : g_err.c_str(); }
 
+int fgl_trim(int32_t device) {
+    if (device < -1) return FGL_E_INVALID;
+    pool_empty(device);
+    stages_empty();
+    return FGL_OK;
+}
+
 int fgl_ctx_create(int32_t width, int32_t height, fgl_ctx **out) {
     if (!out || width <= 0 || height <= 0 || (int64_t)width * height > ((int64_t)1 << 31)) {
         set_err(g_err, "fgl_ctx_create: invalid size %d x %d", width, height);
@@ -1169,7 +1186,13 @@ int fgl_texture_create(fgl_ctx *ctx, int32_t width, int32_t height, int32_t kind
         return FGL_E_INVALID;
     }
     size_t bytes = (size_t)width * height * (kind == FGL_TEX_RGBA16 ? 8 : 4);
-    Tex t;
+    const int64_t h = ctx->next_tex;
+    Tex &t = ctx->tex[h];
+    auto drop = [&](hipError_t e, const char *what) {
+        ctx->tex.erase(h);
+        set_err(ctx->err, "%s failed: %s", what, hipGetErrorString(e));
+        return FGL_E_DEVICE;
+    };
     t.w = width;
     t.h = height;
     t.kind = kind;
@@ -1180,16 +1203,11 @@ int fgl_texture_create(fgl_ctx *ctx, int32_t width, int32_t height, int32_t kind
     } else {
         for (size_t k = 0; k < ntexel && t.solid; k++) t.solid = static_cast<const uint8_t *>(texels)[4 * k + 3] != 0;
     }
-    HIPCHK(ctx, hipSetDevice(ctx->device));
-    HIPCHK(ctx, hipMalloc(&t.d, bytes));
-    hipError_t e = hipMemcpy(t.d, texels, bytes, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        (void)hipFree(t.d);
-        set_err(ctx->err, "texture upload failed: %s", hipGetErrorString(e));
-        return FGL_E_DEVICE;
-    }
-    int64_t h = ctx->next_tex++;
-    ctx->tex[h] = t;
+    hipError_t e = hipSetDevice(ctx->device);
+    if (e != hipSuccess) return drop(e, "hipSetDevice");
+    if ((e = t.d.ensure(bytes)) != hipSuccess) return drop(e, "texture allocation");
+    if ((e = hipMemcpy(t.d.p, texels, bytes, hipMemcpyHostToDevice)) != hipSuccess) return drop(e, "texture upload");
+    ctx->next_tex++;
     *handle = h;
     return FGL_OK;
 }
@@ -1201,9 +1219,8 @@ int fgl_texture_destroy(fgl_ctx *ctx, int64_t handle) {
         ctx->err = "fgl_texture_destroy: unknown handle";
         return FGL_E_INVALID;
     }
+    (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
-    (void)hipFree(it->second.d);
-    g_dev_epoch++;
     ctx->tex.erase(it);
     return FGL_OK;
 }

@@ -118,6 +118,13 @@ typedef struct fgl_mesh fgl_mesh;
  * device 0 when this was never called.  No reference counterpart. */
 int fgl_init(int32_t device);
 
+/* Gives back what the library keeps for its next objects of memory that its
+ * earlier ones have let go: device memory of `device` (-1: of every device),
+ * at most 512 MiB in all, and the page-locked buffers of readbacks, 16 MiB.
+ * The library does so itself before an allocation of its own is refused; this
+ * is for other allocators in the process.  No reference counterpart. */
+int fgl_trim(int32_t device);
+
 /* Message for the last failure on ctx, or the last failure without a
  * context when ctx is NULL.  Never returns NULL. */
 const char *fgl_last_error(const fgl_ctx *ctx);

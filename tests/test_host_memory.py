@@ -25,3 +25,54 @@ ctx.close()
 assert fake.fake_last_error() == 0
 assert fake.fake_live() < live  # freed all the same, and not kept
 """)
+
+
+def test_kept_memory_is_given_back_before_a_texture_is_refused():
+    host_only.run(SETUP + """
+before = fake.fake_live()
+big = [A.NewContext(2000, 1500) for _ in range(4)]
+for c in big:
+    c.close()
+kept = fake.fake_live() - before
+assert kept >= 4 * 12 * 2000 * 1500, kept
+# room for the texture only without what is kept
+fake.fake_limit(fake.fake_live() + (1 << 20))
+tex = A.NewImageTexture(np.full((2048, 1024, 4), 255, dtype=np.uint8), "NRGBA")
+ctx.Shader = A.NewTextureShader(A.Identity(), tex)
+ctx.DrawTriangles(soup(10))  # uploads the texture
+assert fake.fake_last_error() == 0
+# refused where there is no room even so, and nothing is left of the attempt
+live = fake.fake_live()
+fake.fake_limit(live + (1 << 20))
+ctx.Shader = A.NewTextureShader(A.Identity(), A.NewImageTexture(np.full((2048, 2048, 4), 255, dtype=np.uint8), "NRGBA"))
+try:
+    ctx.DrawTriangles(soup(10))
+    raise SystemExit("not refused")
+except N.FglError:
+    pass
+fake.fake_limit(ctypes.c_size_t(-1).value)
+ctx.DrawTriangles(soup(10))
+""")
+
+
+def test_trim_gives_everything_kept_back():
+    host_only.run(SETUP + """
+before = fake.fake_live()
+c = A.NewContext(300, 200)
+c.Image()
+c.close()
+assert fake.fake_live() > before
+A.TrimMemory()
+assert fake.fake_live() == before
+A.TrimMemory()
+""")
+
+
+def test_kept_memory_is_bounded():
+    host_only.run(SETUP + """
+for bound, size, count in ((512 << 20, (2560, 1440), 40), (512 << 20, (64, 64), 300)):
+    cs = [A.NewContext(*size) for _ in range(count)]
+    for c in cs:
+        c.close()
+    assert fake.fake_live() <= bound + (1 << 20), fake.fake_live()
+""")
