@@ -149,6 +149,15 @@ struct DevBuf {
         p = nullptr;
         bytes = 0;
     }
+    // For a buffer whose users have been waited for and whose address no
+    // recorded launch holds: no wait, and recorded batches stay valid.
+    void retire() {
+        if (!p) return;
+        if (bytes <= kPoolBlock) pool_put(dev, p, bytes);
+        else (void)hipFree(p);
+        p = nullptr;
+        bytes = 0;
+    }
     hipError_t ensure(size_t need) {
         if (need <= bytes && p) return hipSuccess;
         release();
@@ -406,8 +415,8 @@ struct fgl_ctx {
     ResolveTent4 rs_t4{};              // the tables as packed uniform 4x weights, when they are
     hipEvent_t xev = nullptr;          // orders another context's stream after this one
     DevBuf dpart, dimg;
-    DevBuf png;    // EncodePNG's workspace
-    HostBuf hpng;  // the encoded stream's size and checksums as the host reads them back
+    DevBuf png;    // the size and checksums of EncodePNG's stream
+    HostBuf hpng;  // the same as the host reads them back
     uint32_t side_rec_cap = 0, side_vtx_cap = 0, pair_cap = 0;
     DrawCounters last{};
 
@@ -2778,42 +2787,63 @@ int fgl_encode_png(fgl_ctx *ctx, uint8_t *out, int64_t cap, int64_t *len) {
     int r = materialize(c, CB_COLOR);
     if (r) return r;
     const int32_t W = c->W, H = c->H;
-    // one workspace, kept with the context and sized for four bytes a pixel:
-    // result, pieces' records, offsets, filtered stream (whole pieces),
-    // pieces' words, packed stream
-    const int64_t np = ((int64_t)H * ((int64_t)W * 4 + 1) + PNG_CHUNK - 1) / PNG_CHUNK;
-    const size_t words_bytes = (size_t)np * PNG_CAP_WORDS * 4;
+    // One workspace for the call: pieces' records, offsets, filtered stream
+    // (whole pieces), pieces' words, packed stream.  Sized for four bytes a
+    // pixel and the longest packed stream (13 bytes a pixel) it spares the
+    // device two reads back, and its block is kept for the next call; where
+    // that is more than the blocks that are kept, it is sized by what the
+    // device has found: 6.4 bytes a pixel (opaque) or 8.5, and the packed stream.
     auto up = [](size_t n) { return (n + 255) / 256 * 256; };
-    const size_t o_rec = 256, o_offs = o_rec + up((size_t)np * sizeof(PngPiece)), o_str = o_offs + up((size_t)np * 8),
-                 o_words = o_str + (size_t)np * PNG_CHUNK, o_pack = o_words + up(words_bytes);
-    HIPCHK(c, c->png.ensure(o_pack + words_bytes));
+    auto pieces = [&](int bpp) { return ((int64_t)H * ((int64_t)W * bpp + 1) + PNG_CHUNK - 1) / PNG_CHUNK; };
+    auto words_bytes = [](int64_t np) { return (size_t)np * PNG_CAP_WORDS * 4; };
+    auto bytes = [&](int64_t np) {
+        return up((size_t)np * sizeof(PngPiece)) + up((size_t)np * 8) + (size_t)np * PNG_CHUNK + up(words_bytes(np));
+    };
+    int64_t np = pieces(4);
+    const bool exact = bytes(np) + words_bytes(np) > kPoolBlock;
+    HIPCHK(c, c->png.ensure(sizeof(PngResult)));
     HIPCHK(c, c->hpng.ensure(sizeof(PngResult)));
-    uint8_t *ws = c->png.as<uint8_t>();
-    PngResult *res = reinterpret_cast<PngResult *>(ws);
-    PngPiece *rec = reinterpret_cast<PngPiece *>(ws + o_rec);
-    uint8_t *packed = ws + o_pack;
+    PngResult *res = c->png.as<PngResult>();
+    auto read_result = [&] {
+        const hipError_t e = hipMemcpyAsync(c->hpng.p, res, sizeof(PngResult), hipMemcpyDeviceToHost, c->stream);
+        return e != hipSuccess ? e : wait_stream(c->stream);
+    };
     HIPCHK(c, hipMemsetAsync(res, 0, sizeof(PngResult), c->stream));
     if ((r = launch(c, "png_opaque", [&] {
              return launch_png_opaque(c->color.as<uint32_t>(), (int64_t)W * H, res, c->stream);
          })))
         return r;
+    if (exact) {
+        HIPCHK(c, read_result());
+        np = pieces(c->hpng.as<PngResult>()->translucent ? 4 : 3);
+    }
+    DevBuf ws, exact_pack;
+    HIPCHK(c, ws.ensure(bytes(np) + (exact ? 0 : words_bytes(np))));
+    PngPiece *rec = ws.as<PngPiece>();
+    uint64_t *offs = reinterpret_cast<uint64_t *>(ws.as<uint8_t>() + up((size_t)np * sizeof(PngPiece)));
+    uint8_t *filtered = reinterpret_cast<uint8_t *>(offs) + up((size_t)np * 8);
+    uint32_t *words = reinterpret_cast<uint32_t *>(filtered + (size_t)np * PNG_CHUNK);
+    uint8_t *packed = ws.as<uint8_t>() + bytes(np);
     // image/png: RGBA unless NRGBA.Opaque(); the kernels read the flag
     if ((r = launch(c, "png_filter", [&] {
-             return launch_png_filter(c->color.as<uint32_t>(), W, H, res, ws + o_str, c->stream);
+             return launch_png_filter(c->color.as<uint32_t>(), W, H, res, filtered, c->stream);
          })))
         return r;
     if ((r = launch(c, "png_deflate", [&] {
-             return launch_png_deflate(ws + o_str, W, H, res, np, reinterpret_cast<uint32_t *>(ws + o_words), rec,
-                                       c->stream);
+             return launch_png_deflate(filtered, W, H, res, np, words, rec, c->stream);
          })))
         return r;
+    if ((r = launch(c, "png_scan", [&] { return launch_png_scan(rec, W, H, res, offs, c->stream); }))) return r;
+    if (exact) {
+        HIPCHK(c, read_result());
+        HIPCHK(c, exact_pack.ensure((size_t)c->hpng.as<PngResult>()->total));
+        packed = exact_pack.as<uint8_t>();
+    }
     if ((r = launch(c, "png_pack", [&] {
-             return launch_png_pack(reinterpret_cast<uint32_t *>(ws + o_words), rec, W, H, np, res,
-                                    reinterpret_cast<uint64_t *>(ws + o_offs), packed, c->stream);
+             return launch_png_pack(words, rec, offs, W, H, np, res, packed, c->stream);
          })))
         return r;
-    HIPCHK(c, hipMemcpyAsync(c->hpng.p, res, sizeof(PngResult), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, wait_stream(c->stream));
+    HIPCHK(c, read_result());
     const PngResult pr = *c->hpng.as<PngResult>();
     const int32_t bpp = pr.translucent ? 4 : 3;
     const uint64_t total = pr.total;
@@ -2838,6 +2868,8 @@ int fgl_encode_png(fgl_ctx *ctx, uint8_t *out, int64_t cap, int64_t *len) {
     z[0] = 0x78;  // deflate, 32K window
     z[1] = 0x9C;  // default level, header check
     HIPCHK(c, copy_out(c->device, z + 2, packed, (size_t)total, c->stream));
+    ws.retire();
+    exact_pack.retire();
     z[2 + total] = 0x03;  // final block: fixed codes, end of block only
     z[3 + total] = 0x00;
     put_be32(z + 4 + total, pr.adler);

@@ -297,9 +297,11 @@ hipError_t launch_png_filter(const uint32_t *color, int32_t W, int32_t H, const 
                              hipStream_t s);
 hipError_t launch_png_deflate(const uint8_t *stream, int32_t W, int32_t H, const PngResult *res, int64_t npieces,
                               uint32_t *out, PngPiece *pieces, hipStream_t s);
-// the pieces back to back in dst, offs their offsets; res: the stream's size and checksums
-hipError_t launch_png_pack(const uint32_t *words, const PngPiece *pieces, int32_t W, int32_t H, int64_t npieces,
-                           PngResult *res, uint64_t *offs, uint8_t *dst, hipStream_t s);
+// the pieces' offsets in the stream; res: its size and Adler-32
+hipError_t launch_png_scan(const PngPiece *pieces, int32_t W, int32_t H, PngResult *res, uint64_t *offs, hipStream_t s);
+// the pieces back to back in dst; res: the stream's CRC-32
+hipError_t launch_png_pack(const uint32_t *words, const PngPiece *pieces, const uint64_t *offs, int32_t W, int32_t H,
+                           int64_t npieces, PngResult *res, uint8_t *dst, hipStream_t s);
 // CRC-32 register after n bytes whose register from 0 is raw, following state
 uint32_t png_crc_append(uint32_t state, uint32_t raw, uint64_t n);
 

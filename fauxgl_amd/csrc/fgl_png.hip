@@ -814,11 +814,13 @@ hipError_t launch_png_deflate(const uint8_t *stream, int32_t W, int32_t H, const
     hipLaunchKernelGGL(k_png_deflate, dim3((unsigned)npieces), dim3(PD_THREADS), 0, s, stream, W, H, res, out, pieces);
     return hipGetLastError();
 }
-hipError_t launch_png_pack(const uint32_t *words, const PngPiece *pieces, int32_t W, int32_t H, int64_t npieces,
-                           PngResult *res, uint64_t *offs, uint8_t *dst, hipStream_t s) {
+hipError_t launch_png_scan(const PngPiece *pieces, int32_t W, int32_t H, PngResult *res, uint64_t *offs,
+                           hipStream_t s) {
     hipLaunchKernelGGL(k_png_scan, dim3(1), dim3(PS_THREADS), 0, s, pieces, W, H, res, offs);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    return hipGetLastError();
+}
+hipError_t launch_png_pack(const uint32_t *words, const PngPiece *pieces, const uint64_t *offs, int32_t W, int32_t H,
+                           int64_t npieces, PngResult *res, uint8_t *dst, hipStream_t s) {
     hipLaunchKernelGGL(k_png_pack, dim3((unsigned)npieces), dim3(256), 0, s, words, pieces, offs, W, H, res, dst);
     return hipGetLastError();
 }

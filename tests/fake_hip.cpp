@@ -169,7 +169,11 @@ namespace {
 hipError_t draw(const DrawArgs &, hipStream_t) { return hipSuccess; }
 hipError_t pass(const DrawArgs &, int, hipStream_t) { return hipSuccess; }
 uint32_t one_block(int, const DrawArgs &, bool) { return 1; }
-hipError_t many(int, const MultiArgs &, uint32_t, const DrawArgs &, hipStream_t) { return hipSuccess; }
+long multi = 0;  // launches of replayed batches
+hipError_t many(int, const MultiArgs &, uint32_t, const DrawArgs &, hipStream_t) {
+    multi++;
+    return hipSuccess;
+}
 template <class F>
 void set(F &slot) {
     if constexpr (std::is_convertible_v<decltype(&draw), F>) slot = draw;
@@ -194,3 +198,9 @@ TileOps ops(int w, int h) {
     }
 FGL_TILE_SHAPES(FAKE_OPS)
 }  // namespace fgl
+
+extern "C" long fake_count_multi() {
+    const long n = fgl::multi;
+    fgl::multi = 0;
+    return n;
+}

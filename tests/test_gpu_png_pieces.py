@@ -86,5 +86,28 @@ def test_pieces(name):
     ctx.SetColorBuffer(img)
     _, want = O.png_filter(img)
     z, _ = png_ref.zlib_stream(want)
-    for _ in range(2):  # the workspace is kept
+    for _ in range(2):  # the second in a kept workspace
         assert chunks(ctx.EncodePNG())[1][1] == z
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("alpha", [255, 254])
+@pytest.mark.parametrize("h", [2500, 2560])
+def test_workspace_sizes(h, alpha):
+    """Frames on both sides of the size (10.3 Mpixel) above which the workspace
+    is sized by what the device has found and is not kept."""
+    import zlib
+    print(f"[case] png workspace 4096x{h} alpha {alpha}", flush=True)
+    rng = np.random.Generator(np.random.PCG64(h))
+    img = rng.integers(0, 256, (h, 4096, 4), dtype=np.uint8)
+    img[:, 1000:] //= 200  # long runs
+    img[..., 3] = 255
+    img[h - 1, 4095, 3] = alpha
+    ctx = A.NewContext(4096, h)
+    ctx.SetColorBuffer(img)
+    bpp, want = O.png_filter(img)
+    assert bpp == (3 if alpha == 255 else 4)
+    first = ctx.EncodePNG()
+    assert zlib.decompress(chunks(first)[1][1]) == want.tobytes()
+    assert ctx.EncodePNG() == first
+    ctx.close()

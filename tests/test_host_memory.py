@@ -76,3 +76,50 @@ for bound, size, count in ((512 << 20, (2560, 1440), 40), (512 << 20, (64, 64), 
         c.close()
     assert fake.fake_live() <= bound + (1 << 20), fake.fake_live()
 """)
+
+
+def test_encoding_a_png_keeps_no_memory_in_the_context():
+    """The workspace is kept as other freed blocks are, where it is one they
+    take; a larger one is freed, and is no larger than the image needs (the
+    fake device finds an opaque image and an empty stream)."""
+    host_only.run(SETUP + """
+c = A.NewContext(800, 600)
+c.EncodePNG()
+A.TrimMemory()
+before = fake.fake_live()
+c.EncodePNG()
+assert before < fake.fake_live() < before + 13.2 * 800 * 600
+n = fake.fake_mallocs()
+c.EncodePNG()
+assert fake.fake_mallocs() == n
+A.TrimMemory()
+assert fake.fake_live() == before
+c.close()
+c = A.NewContext(7680, 4320)
+c.Image()
+A.TrimMemory()
+before = fake.fake_live()
+fake.fake_peak()
+c.EncodePNG()
+A.TrimMemory()
+assert fake.fake_live() <= before + 256, fake.fake_live() - before
+assert fake.fake_peak() <= before + 6.45 * 7680 * 4320, (fake.fake_peak() - before) / (7680 * 4320)
+""")
+
+
+def test_encoding_a_png_leaves_recorded_batches_valid():
+    """No buffer that a recorded batch uses is freed by it: the next run
+    replays instead of drawing every view again (which would read counters
+    back for each)."""
+    host_only.run(SETUP + """
+dm = ctx.Upload(A.Mesh(soup(100)))
+ctx.Shader = A.NewSolidColorShader(A.Identity(), A.Black)
+b = A.Batch()
+b.Add(ctx, dm)
+b.Run()
+ctx.EncodePNG()
+fake.fake_count_multi.restype = ctypes.c_long
+fake.fake_count_multi()
+b.Run()
+assert fake.fake_count_multi() > 0  # replayed
+""")
