@@ -60,7 +60,8 @@ struct DrawArgs {
     // coverage spans
     uint32_t *pspans;           // spans per sorted pair
     uint16_t *prows;            // per sorted pair: its rows that have spans (ROWS_ALL: every row)
-    uint64_t *span_blocksum;    // per SPAN_GROUP pairs
+    uint32_t *span_groupsum;    // per SPAN_GROUP pairs
+    uint64_t *span_blocksum;    // per SPAN_THREADS pairs
     uint64_t *span_blockoff;
     Span *spans;
     uint32_t span_cap;
