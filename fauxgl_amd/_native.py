@@ -38,7 +38,7 @@ EXPORTED = [
     "fgl_encode_png_bound", "fgl_encode_png",
     "fgl_batch_create", "fgl_batch_destroy", "fgl_batch_error", "fgl_batch_add", "fgl_batch_run",
     "fgl_tile_shapes", "fgl_ctx_set_tile", "fgl_ctx_get_tile", "fgl_autotune_mesh", "fgl_tune_save",
-    "fgl_tune_load", "fgl_tune_clear", "fgl_ctx_force_capacities", "fgl_trim",
+    "fgl_tune_load", "fgl_tune_clear", "fgl_ctx_force_capacities", "fgl_trim", "fgl_draw_depth_first",
 ]
 
 _d = ctypes.c_double
@@ -96,6 +96,7 @@ def load():
     sigs = {
         "fgl_init": (i32, [i32]),
         "fgl_trim": (i32, [i32]),
+        "fgl_draw_depth_first": (i32, [vp, ctypes.POINTER(i32)]),
         "fgl_last_error": (ctypes.c_char_p, [vp]),
         "fgl_ctx_create": (i32, [i32, i32, vpp]),
         "fgl_ctx_destroy": (None, [vp]),

@@ -933,6 +933,13 @@ class Context:
         N.check(N.load().fgl_draw_stats(self._ptr(), ctypes.byref(st)), self._ptr())
         return {name: int(getattr(st, name)) for name, _ in N.FglDrawStat._fields_}
 
+    def DepthFirst(self):
+        """Whether the last draw tested its fragments before shading them; a
+        diagnostic with no reference counterpart."""
+        out = ctypes.c_int32()
+        N.check(N.load().fgl_draw_depth_first(self._ptr(), ctypes.byref(out)), self._ptr())
+        return bool(out.value)
+
 
 def TileShapes():
     """The compiled tile shapes as (w, h) pairs."""

@@ -117,7 +117,7 @@ struct DrawCounters {
     uint32_t spans_lo, spans_hi; // unclamped span count
     uint32_t nfrags;             // fragments (clamped to capacity)
     uint32_t frags_lo, frags_hi; // unclamped fragment count
-    uint32_t zfirst;             // k_zshade draws (DrawArgs::zpick)
+    uint32_t zfirst;             // k_zshade draws (set before it where it need not be: DrawArgs::zpick)
     // UpdatedPixels in UPD_PARTS partial sums (tile t adds into t % UPD_PARTS,
     // spreading the atomics over as many addresses); the host adds them up
     uint32_t upd[64];

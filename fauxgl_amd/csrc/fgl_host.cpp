@@ -1877,6 +1877,16 @@ int fgl_draw_stats(fgl_ctx *ctx, fgl_draw_stat *out) {
     return FGL_OK;
 }
 
+int fgl_draw_depth_first(fgl_ctx *ctx, int32_t *out) {
+    if (check_ctx(ctx)) return FGL_E_INVALID;
+    if (!out) {
+        ctx->err = "fgl_draw_depth_first: null argument";
+        return FGL_E_INVALID;
+    }
+    *out = ctx->last.zfirst != 0;
+    return FGL_OK;
+}
+
 int fgl_ctx_force_capacities(fgl_ctx *ctx, const uint32_t caps[5]) {
     if (check_ctx(ctx)) return FGL_E_INVALID;
     if (!caps) {

@@ -963,6 +963,7 @@ FGL_D void zshade_body(const DrawArgs &a, const G &g) {
         a.ctr->frags_lo = (uint32_t)total;
         a.ctr->frags_hi = (uint32_t)(total >> 32);
         a.ctr->total = total;
+        a.ctr->zfirst = 1u;
     }
     if (total > a.frag_lim) return;
 

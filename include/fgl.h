@@ -353,6 +353,9 @@ typedef struct fgl_draw_stat {
     uint64_t overflow_mask, reruns;
 } fgl_draw_stat;
 int fgl_draw_stats(fgl_ctx *ctx, fgl_draw_stat *out);
+/* Whether the last draw tested its fragments' depths before shading them (1)
+ * or shaded every fragment first (0): a diagnostic, the results are the same. */
+int fgl_draw_depth_first(fgl_ctx *ctx, int32_t *out);
 
 /* Failure injection (no reference counterpart; for tests of the capacity
  * path).  The next triangle or line draw on ctx starts its first pass with

@@ -121,3 +121,86 @@ def test_mixed_kernel_variants_equal_single_draws():
                 assert np.array_equal(c.Image(), wimg), (rep, k)
                 assert np.array_equal(c.DepthBuffer.view(np.uint64), wdepth.view(np.uint64)), (rep, k)
     b.close()
+
+
+def _deep(n, seed, extent):
+    rng = np.random.Generator(np.random.PCG64(seed))
+    c = rng.uniform(-1, 1, size=(n, 1, 3)) * [1, 1, 0.8]
+    pos = np.clip(c + rng.uniform(-extent, extent, size=(n, 3, 3)) * [1, 1, 0.1], -1, 1)
+    return A.Prims(pos, M.with_face_normals(pos), rng.uniform(0, 1, size=(n, 3, 2)))
+
+
+# (size, soup, shader, state, depth first): fragments tested before they are
+# shaded in every variant the others of a batch must not share a launch with
+# (color written or not, opaque or blended, the device's choice both ways), and
+# shaded first.  1600x1504 is 2350 tiles.  "shared" views follow each other on
+# one context, "empty" is a view without primitives.
+TESTED = [
+    ((97, 67), "small", "phong", {}, True),
+    ((97, 67), "small", "phong", {"WriteColor": False}, True),
+    ((97, 67), "small", "blend", {}, True),
+    ((97, 67), "small", "blend", {"WriteColor": False}, True),
+    ((97, 67), "small", "solid", {"WriteColor": False, "WriteDepth": False}, True),
+    ((97, 67), "small", "discard", {}, False),
+    ((1600, 1504), "deep", "phong", {}, True),
+    ((1600, 1504), "shallow", "phong", {}, False),
+    ((1600, 1504), "deep", "blend", {}, True),
+    ((1600, 1504), "shallow", "blend", {}, False),
+    ((1600, 1504), "deep", "phong", {"WriteColor": False}, True),
+    ("shared", "small", "discard", {}, False),
+    ("shared", "large", "solid", {}, True),
+    ("shared", "small", "blend", {"WriteColor": False}, True),
+]
+
+
+@pytest.mark.parametrize("empty", [False, True])  # with an empty view the batch is a recorded graph
+def test_tested_first_equals_the_oracle(empty):
+    import oracle as O
+    from helpers import compare, oracle_shader
+    _say(f"batch of draws tested first and not, graph {empty}, 4 runs")
+    home = A.NewContext(8, 8)
+    soups = {"small": _deep(60, 1, 0.6), "large": _deep(400, 2, 0.3), "deep": _deep(60, 4, 0.9),
+             "shallow": _deep(40, 5, 0.1)}
+    light, eye = A.V(0.2, 0.4, 1).Normalize(), A.V(0, 0, 3)
+    shaders = {"phong": A.PhongShader(A.Identity(), light, eye, A.Color(0.3, 0.6, 0.4, 1.0)),
+               "blend": A.PhongShader(A.Identity(), light, eye, A.Color(0.3, 0.6, 0.4, 0.4)),
+               "solid": A.NewSolidColorShader(A.Identity(), A.Color(0.2, 0.4, 0.6, 1.0)),
+               "discard": A.NewSolidColorShader(A.Identity(), A.Discard)}
+    meshes = {k: home.Upload(A.Mesh(p)) for k, p in soups.items()}
+    shared = A.NewContext(120, 90)
+    b, ctxs, want = A.Batch(), [], []
+    if empty:
+        c = A.NewContext(40, 30)
+        c.Shader = shaders["solid"]
+        b.Add(c, home.Upload(A.Mesh(A.Prims(np.zeros((0, 3, 3))))), clear_color=M.BACKGROUND)
+        ctxs.append(c)
+        want.append(None)
+    for size, soup, shader, state, _ in TESTED:
+        c = shared if size == "shared" else A.NewContext(*size)
+        c.Shader, c.Cull = shaders[shader], A.CullNone
+        c.WriteColor, c.WriteDepth = state.get("WriteColor", True), state.get("WriteDepth", True)
+        b.Add(c, meshes[soup], clear_color=M.BACKGROUND)
+        ctxs.append(c)
+        o = O.Context(c.Width, c.Height)
+        o.clear_color(tuple(M.BACKGROUND))
+        o.clear_depth(A.MaxFloat64)
+        o.set_state(O.make_state(front_face=O.FACE_CCW, line_width=2.0, read_depth=True, write_depth=c.WriteDepth,
+                                 write_color=c.WriteColor, alpha_blend=True, wireframe=False, cull=A.CullNone,
+                                 depth_bias=0.0))
+        o.set_shader(oracle_shader(c.Shader))
+        info = o.draw_triangles(O.Mesh(tris=soups[soup].arrays()), 1)
+        want.append((o.color(), o.depth(), [info]))
+    last_on = {id(c): k for k, c in enumerate(ctxs)}
+    for rep in range(4):
+        infos = b.Run()
+        for k, c in enumerate(ctxs):
+            if want[k] is None or last_on[id(c)] != k:
+                continue
+            case = TESTED[k - empty]
+            res = compare(want[k], (c.Image(), c.DepthBuffer, [tuple(infos[k])]), color_tol=0)
+            assert res["ok"], (rep, case, res)
+            assert c.DepthFirst() == case[4], (rep, case)
+        for c in set(ctxs):  # scribble on the framebuffers between the runs
+            c.ClearColorBufferWith(A.Color(1, 0, 0, 1))
+            c.Image()
+    b.close()

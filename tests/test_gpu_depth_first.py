@@ -54,9 +54,10 @@ _FIELDS = {"ReadDepth": "read_depth", "WriteDepth": "write_depth", "WriteColor":
            "AlphaBlend": "alpha_blend", "Wireframe": "wireframe", "Cull": "cull", "DepthBias": "depth_bias"}
 
 
-def _check(name, shader, W, H, draws, states, tile=None):
+def _check(name, shader, W, H, draws, states, tile=None, first=None):
     """Clears, then the draws each with its state, in both; a second frame on
-    the same context follows with the clears pending again."""
+    the same context follows with the clears pending again.  first(state):
+    whether a draw is to be tested before it is shaded."""
     _say(f"depth first: {name}")
     octx, gctx = O.Context(W, H), A.NewContext(W, H)
     if tile:
@@ -80,6 +81,8 @@ def _check(name, shader, W, H, draws, states, tile=None):
             m = O.Mesh(tris=prims.arrays())
             ri.append(octx.draw_triangles(m, 1))
             gi.append(tuple(gctx.DrawTriangles(prims)))
+            if first is not None:
+                assert gctx.DepthFirst() == first(full), full
         res = compare((octx.color(), octx.depth(), ri), (gctx.Image(), gctx.DepthBuffer, gi), color_tol=0)
         assert res["ok"], res
     return gctx
@@ -102,7 +105,13 @@ STATES = {
 @pytest.mark.parametrize("shader", list(SHADERS))
 def test_states_and_shaders(shader, state):
     draws = [_soup(60, 1, 0.7), _soup(60, 2, 0.3)]
-    _check(f"{shader}, {state}", SHADERS[shader](), 97, 67, draws, STATES[state])
+
+    def first(st):
+        if shader in ("solid discard", "texture with a hole"):
+            return False
+        # without a depth test blended fragments are shaded as they come
+        return st["ReadDepth"] or not (st["AlphaBlend"] and st["WriteColor"]) or shader in ("solid", "phong")
+    _check(f"{shader}, {state}", SHADERS[shader](), 97, 67, draws, STATES[state], first=first)
 
 
 @pytest.mark.gpu
@@ -110,7 +119,8 @@ def test_states_and_shaders(shader, state):
 @pytest.mark.parametrize("shader", ["phong", "texture", "solid translucent"])
 def test_tile_shapes(shader, tile):
     # 900 large triangles: hundreds of fragments a pixel, mostly behind
-    _check(f"{shader}, {tile}", SHADERS[shader](), 257, 131, [_soup(900, 3, 0.9)], [{}], tile)
+    _check(f"{shader}, {tile}", SHADERS[shader](), 257, 131, [_soup(900, 3, 0.9)], [{}], tile,
+           first=lambda st: tile[0] * tile[1] <= 2048)
 
 
 @pytest.mark.gpu
@@ -122,6 +132,7 @@ def test_many_tiles(shader, size, deep):
     prims = _soup(60, 4, 0.9) if deep else _soup(40, 5, 0.1)
     ctx = _check(f"{shader}, {W}x{H}, deep {deep}", SHADERS[shader](), W, H, [prims], [{}])
     assert (ctx.DrawStats()["fragments"] >= 2 * W * H) == deep
+    assert ctx.DepthFirst() == (deep or W * H < 2304 * 1024)
 
 
 @pytest.mark.gpu
@@ -133,6 +144,7 @@ def test_dense_triangles(n, deep):
     prims = _soup(n, 6, 0.03 if deep else 0.004)
     ctx = _check(f"{n} triangles, deep {deep}", SHADERS["phong"](), W, H, [prims], [{}])
     assert (ctx.DrawStats()["fragments"] >= 2 * W * H) == deep
+    assert ctx.DepthFirst() == (deep or n == 102400)
 
 
 @pytest.mark.gpu
@@ -168,5 +180,6 @@ def test_forced_fragment_overflow(shader, size, n):
             gi.append(tuple(ctx.DrawTriangles(p)))
         st = ctx.DrawStats()
         assert st["overflow_mask"] == 32 and st["reruns"] == 1, st
+        assert ctx.DepthFirst() == (shader != "texture with a hole")
         res = compare((octx.color(), octx.depth(), ri), (ctx.Image(), ctx.DepthBuffer, gi), color_tol=0)
         assert res["ok"], res
