@@ -16,6 +16,7 @@ raises (the reference's Go CPU path is what serves custom shaders).
 import ctypes
 import os
 import math
+import weakref
 from collections import namedtuple
 
 import numpy as np
@@ -306,18 +307,17 @@ class ImageTexture:
             raise ValueError("texels must be (H, W, 4)")
         self.Height, self.Width = self.Image.shape[:2]
         self.kind = kind
-        self._handles = {}
+        self._handles = weakref.WeakKeyDictionary()  # per Context; gone with it
 
     def handle(self, ctx):
         ptr = ctx._ptr()
-        key = ptr.value
-        h = self._handles.get(key)
+        h = self._handles.get(ctx)
         if h is None:
             out = ctypes.c_int64(0)
             N.check(N.load().fgl_texture_create(ptr, self.Width, self.Height, self._kinds[self.kind],
                                                 self.Image.ctypes.data_as(ctypes.c_void_p), ctypes.byref(out)), ptr)
             h = out.value
-            self._handles[key] = h
+            self._handles[ctx] = h
             ctx._textures.append(self)
         return h
 
