@@ -117,13 +117,15 @@ struct DrawCounters {
     uint32_t spans_lo, spans_hi; // unclamped span count
     uint32_t nfrags;             // fragments (clamped to capacity)
     uint32_t frags_lo, frags_hi; // unclamped fragment count
-    uint32_t zfirst;             // k_zshade draws (set before it where it need not be: DrawArgs::zpick)
+    uint32_t zfirst;             // k_zshade draws or drew
     // UpdatedPixels in UPD_PARTS partial sums (tile t adds into t % UPD_PARTS,
     // spreading the atomics over as many addresses); the host adds them up
     uint32_t upd[64];
     // fragments in 64 partial sums (DrawArgs::zmode; span waves add into
     // part wave % 64)
     unsigned long long ftot[64];
+    uint32_t crowded;            // a tile holds too large a part of the spans (DrawArgs::crowd_min)
+    uint32_t pad3;
 };
 constexpr int UPD_PARTS = 64;
 // DrawCounters::overflow: fragments past the capacity.  The kernels that find

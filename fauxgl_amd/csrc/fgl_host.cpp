@@ -805,6 +805,40 @@ int draw_zmode(const DrawArgs &a) {
     return a.st.read_depth ? 2 : 0;
 }
 
+// The rest of how a draw that can be tested first is drawn (the measurements
+// are at k_zshade).  picked: for a recorded draw, whether its last direct run
+// was tested first.
+void draw_zpick(DrawArgs &a, int kind, const bool *picked) {
+    // raster triangles (a line is two, and wireframe draws three lines)
+    const int64_t n = a.in.n * (kind == PRIM_LINE ? 2 : a.st.wireframe ? 6 : 1);
+    const bool few = a.ntiles <= ZTILES_FEW;
+    const bool large = a.ntiles > ZTILES_DIRECT ||
+                       ((int64_t)a.W * a.H > ZDENSE_PIX && n > (int64_t)ZTILE_DENSE * a.ntiles);
+    a.z512 = few || (!large && (a.zmode == 1 || n <= (int64_t)ZTILE_SPARSE * a.ntiles));
+    if (large) {
+        a.zpick = ZPICK_DEVICE;
+        a.crowd_min = 1280;
+        a.crowd_part = 256;
+    } else if (n > ZPRIMS_DIRECT) {
+        a.zpick = ZPICK_CROWD;
+        const uint32_t f = (a.zmode == 2 ? 2 : 1) * (a.z512 ? 1 : 2);
+        a.crowd_min = 10000 / f;
+        a.crowd_part = 32 * f;
+    }
+    if (a.zpick && picked) {
+        a.zpick = ZPICK_NONE;
+        if (!*picked) a.zmode = 0;
+    }
+}
+
+// Its fragments shaded, then tested and written in order.
+int draw_shade(fgl_ctx *c, const TileOps &T, const DrawArgs &a) {
+    int r;
+    if ((r = launch(c, "frag_scan", [&] { return T.frag_scan(a, c->stream); }))) return r;
+    if ((r = launch(c, "shade", [&] { return T.shade(a, c->stream); }))) return r;
+    return launch(c, "rop", [&] { return T.rop(a, c->stream); });
+}
+
 // One pass of a draw: the kernel sequence on the context's stream.
 int draw_pass(fgl_ctx *c, const TileOps &T, const DrawArgs &a, int kind) {
     int r;
@@ -823,18 +857,17 @@ int draw_pass(fgl_ctx *c, const TileOps &T, const DrawArgs &a, int kind) {
     if ((r = launch(c, "span_count", [&] { return T.span_count(a, c->stream); }))) return r;
     if ((r = launch(c, "span_scan", [&] { return T.span_scan(a, c->stream); }))) return r;
     if ((r = launch(c, "spans", [&] { return T.spans(a, c->stream); }))) return r;
-    if (a.zmode && !a.zpick) return launch(c, "zshade", [&] { return T.zshade(a, c->stream); });
-    if ((r = launch(c, "frag_scan", [&] { return T.frag_scan(a, c->stream); }))) return r;
-    if ((r = launch(c, "shade", [&] { return T.shade(a, c->stream); }))) return r;
-    if ((r = launch(c, "rop", [&] { return T.rop(a, c->stream); }))) return r;
-    return a.zpick ? launch(c, "zshade", [&] { return T.zshade(a, c->stream); }) : FGL_OK;
+    if (a.zmode && a.zpick != ZPICK_DEVICE) return launch(c, "zshade", [&] { return T.zshade(a, c->stream); });
+    if ((r = draw_shade(c, T, a))) return r;
+    return a.zpick == ZPICK_DEVICE ? launch(c, "zshade", [&] { return T.zshade(a, c->stream); }) : FGL_OK;
 }
 
 // The first part of a draw: checks, the shader, the framebuffer and state
 // fields, the starting capacities and the buffers whose size does not depend
 // on them.  An empty draw returns FGL_OK with a.in.n == 0 and T unset.
+// picked: as for draw_zpick.
 int draw_begin(fgl_ctx *c, const fgl_state *st, const fgl_shader *sh, int kind, const DevPrims &in, const TileOps *&T,
-               DrawArgs &a) {
+               DrawArgs &a, const bool *picked = nullptr) {
     if (in.n < 0 || in.n > kMaxPrims) {
         set_err(c->err, "primitive count %lld outside [0, %lld]", (long long)in.n, (long long)kMaxPrims);
         return FGL_E_INVALID;
@@ -849,10 +882,9 @@ int draw_begin(fgl_ctx *c, const fgl_state *st, const fgl_shader *sh, int kind, 
     }
     T = draw_ops(c, kind, in.n);
     draw_setup(c, st, *T, kind, in, a);
-    a.zmode = T->tw * T->th <= ZTILE_PIX ? draw_zmode(a) : 0;
-    a.zpick = a.zmode && (a.ntiles > ZTILES_DIRECT ||
-                          ((int64_t)a.W * a.H > ZDENSE_PIX && in.n > (int64_t)ZTILE_DENSE * a.ntiles));
     const int64_t n = in.n;
+    a.zmode = T->tw * T->th <= ZTILE_PIX ? draw_zmode(a) : 0;
+    if (a.zmode) draw_zpick(a, kind, picked);
 
     // starting capacities; grown on overflow
     uint64_t want_side = kind == PRIM_LINE ? (uint64_t)2 * n : (st->wireframe ? (uint64_t)6 * n : (uint64_t)n / 8);
@@ -955,11 +987,11 @@ int draw_buffers(fgl_ctx *c, DrawArgs &a) {
 }
 
 int run_draw(fgl_ctx *c, const fgl_state *st, const fgl_shader *sh, int kind, const DevPrims &in, uint64_t info[2],
-             uint32_t *capture_ctr = nullptr) {
+             uint32_t *capture_ctr = nullptr, const bool *picked = nullptr) {
     if (info) info[0] = info[1] = 0;
     DrawArgs a;
     const TileOps *Tp = nullptr;
-    int r = draw_begin(c, st, sh, kind, in, Tp, a);
+    int r = draw_begin(c, st, sh, kind, in, Tp, a, picked);
     if (r || in.n == 0) return r;
     const TileOps &T = *Tp;
 
@@ -990,8 +1022,20 @@ int run_draw(fgl_ctx *c, const fgl_state *st, const fgl_shader *sh, int kind, co
             });
 
         HIPCHK(c, c->hctr.ensure(sizeof(DrawCounters)));
-        HIPCHK(c, hipMemcpyAsync(c->hctr.p, a.ctr, sizeof(DrawCounters), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, wait_stream(c->stream));
+        auto read_counters = [&] {
+            const hipError_t e =
+                hipMemcpyAsync(c->hctr.p, a.ctr, sizeof(DrawCounters), hipMemcpyDeviceToHost, c->stream);
+            return e != hipSuccess ? e : wait_stream(c->stream);
+        };
+        HIPCHK(c, read_counters());
+        if (a.zpick == ZPICK_CROWD && c->hctr.as<DrawCounters>()->crowded && !c->hctr.as<DrawCounters>()->overflow) {
+            // the spans and their fragments' offsets are there; nothing is drawn
+            DrawArgs b = a;
+            b.zmode = 0;
+            b.zpick = ZPICK_NONE;
+            if ((r = draw_shade(c, T, b))) return r;
+            HIPCHK(c, read_counters());
+        }
         const DrawCounters h = *c->hctr.as<DrawCounters>();
         if (c->prof) prof_collect(c);
         c->last = h;
@@ -2926,6 +2970,9 @@ struct fgl_batch {
         uint32_t clear_color;
         double clear_depth;
         uint32_t ndeferred = 0;  // triangles its last direct draw queued for clipping
+        // whether its last direct triangle and line draws were tested first: a
+        // replay takes the same way without asking the device
+        bool zfirst[2] = {false, false};
     };
     std::vector<View> views;
     std::vector<fgl_ctx *> ctxs;  // the distinct contexts, in first-use order
@@ -3014,8 +3061,12 @@ int batch_eager(fgl_batch *b, size_t i, uint64_t info[2]) {
     mesh_prims(v.mesh, true, l);
     uint64_t i1[2] = {0, 0}, i2[2] = {0, 0};
     int r = run_draw(v.ctx, &v.st, &v.sh, PRIM_TRI, t, i1);
-    if (!r && t.n > 0) v.ndeferred = v.ctx->last.ndeferred;
+    if (!r && t.n > 0) {
+        v.ndeferred = v.ctx->last.ndeferred;
+        v.zfirst[0] = v.ctx->last.zfirst != 0;
+    }
     if (!r) r = run_draw(v.ctx, &v.st, &v.sh, PRIM_LINE, l, i2);
+    if (!r && l.n > 0) v.zfirst[1] = v.ctx->last.zfirst != 0;
     if (!r && t.n == 0 && l.n == 0) r = materialize(v.ctx);
     if (r) {
         set_err(b->err, "view %zu: %s", i, v.ctx->err.c_str());
@@ -3039,7 +3090,7 @@ int batch_size_buffers(fgl_batch *b) {
             if (p.n == 0) continue;
             DrawArgs a;
             const TileOps *T;
-            int r = draw_begin(v.ctx, &v.st, &v.sh, kind, p, T, a);
+            int r = draw_begin(v.ctx, &v.st, &v.sh, kind, p, T, a, &v.zfirst[kind == PRIM_LINE]);
             if (!r) r = draw_buffers(v.ctx, a);
             if (r) {
                 set_err(b->err, "view %zu: %s", i, v.ctx->err.c_str());
@@ -3087,9 +3138,9 @@ int batch_record(fgl_batch *b) {
         DevPrims t, l;
         mesh_prims(v.mesh, false, t);
         mesh_prims(v.mesh, true, l);
-        r = run_draw(v.ctx, &v.st, &v.sh, PRIM_TRI, t, nullptr, dst + (2 * i) * words);
+        r = run_draw(v.ctx, &v.st, &v.sh, PRIM_TRI, t, nullptr, dst + (2 * i) * words, &v.zfirst[0]);
         if (t.n > 0) v.ctx->pend_color = v.ctx->pend_depth = false;  // the triangle pass clears
-        if (!r) r = run_draw(v.ctx, &v.st, &v.sh, PRIM_LINE, l, nullptr, dst + (2 * i + 1) * words);
+        if (!r) r = run_draw(v.ctx, &v.st, &v.sh, PRIM_LINE, l, nullptr, dst + (2 * i + 1) * words, &v.zfirst[1]);
         if (l.n > 0) v.ctx->pend_color = v.ctx->pend_depth = false;
         if (!r && t.n == 0 && l.n == 0) r = materialize(v.ctx);  // fill kernels: the clear of an empty view
         if (r) set_err(b->err, "view %zu: %s", i, v.ctx->err.c_str());
@@ -3151,7 +3202,7 @@ int batch_record_multi(fgl_batch *b) {
             Item it;
             it.view = i;
             it.kind = kind;
-            int r = draw_begin(v.ctx, &v.st, &v.sh, kind, p, it.T, it.a);
+            int r = draw_begin(v.ctx, &v.st, &v.sh, kind, p, it.T, it.a, &v.zfirst[kind == PRIM_LINE]);
             if (!r) r = draw_buffers(v.ctx, it.a);
             if (r) {
                 set_err(b->err, "view %zu: %s", i, v.ctx->err.c_str());
@@ -3169,10 +3220,10 @@ int batch_record_multi(fgl_batch *b) {
     struct Key {
         int round;
         const TileOps *T;
-        int kind, wire, shk, tex, zmode, zpick, wc;
+        int kind, wire, shk, tex, zmode, wc;
         bool operator<(const Key &o) const {
-            return std::tie(round, T, kind, wire, shk, tex, zmode, zpick, wc) <
-                   std::tie(o.round, o.T, o.kind, o.wire, o.shk, o.tex, o.zmode, o.zpick, o.wc);
+            return std::tie(round, T, kind, wire, shk, tex, zmode, wc) <
+                   std::tie(o.round, o.T, o.kind, o.wire, o.shk, o.tex, o.zmode, o.wc);
         }
     };
     std::map<Key, size_t> gid;
@@ -3186,7 +3237,7 @@ int batch_record_multi(fgl_batch *b) {
             const Item &it = items[k];
             if (it.round != rd) continue;
             const Key key{rd, it.T, it.kind, it.a.st.wireframe ? 1 : 0, it.a.sh.kind, it.a.sh.has_tex ? 1 : 0,
-                          it.a.zmode, it.a.zpick, it.a.st.write_color};
+                          it.a.zmode, it.a.st.write_color};
             auto f = gid.find(key);
             if (f == gid.end()) {
                 f = gid.emplace(key, members.size()).first;
@@ -3255,13 +3306,13 @@ int batch_record_multi(fgl_batch *b) {
         add(ST_SPAN_COUNT, 0);
         add(ST_SPAN_SCAN, 0);
         add(ST_SPANS, 0);
-        const bool zpick = keys[g].zpick != 0;
-        if (!G.rep.zmode || zpick) {
+        if (G.rep.zmode) {
+            add(ST_ZSHADE, 0);
+        } else {
             add(ST_FRAG_SCAN, 0);
             add(ST_SHADE, 0);
             add(ST_ROP, 0);
         }
-        if (G.rep.zmode) add(ST_ZSHADE, 0);
         groups.push_back(std::move(G));
     }
     // each round's counters, gathered into the per-view slots

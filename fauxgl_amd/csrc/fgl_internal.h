@@ -77,8 +77,12 @@ struct DrawArgs {
     // How the fragments are drawn: 0 shaded, then tested and written in order
     // (k_shade, k_rop); where no fragment can be Discard, tested first
     // (k_zshade): 1 every color replaces the pixel's, 2 some may blend.
-    // zpick: the device picks one or the other by the draw's fragments.
+    // zpick: what the device has to say in it (ZPick).
     int32_t zmode, zpick;
+    int32_t z512;               // k_zshade's larger workgroups
+    // A tile is crowded from this many spans on that are also more than one in
+    // crowd_part of the draw's.
+    uint32_t crowd_min, crowd_part;
     uint32_t frag_lim;          // fragments k_zshade draws at most (it stores none)
 
     // framebuffer and deferred clears
@@ -96,14 +100,18 @@ struct DrawArgs {
 };
 
 constexpr int VS_THREADS = 256;
-// Tiles up to which a draw that can be tested first is (see k_zshade): a
-// 1080p frame's, about two rounds of resident workgroups.
-constexpr int ZTILES_DIRECT = 2304;
-// Primitives a tile above which a frame of more than ZDENSE_PIX pixels leaves
-// the choice to the device, and the largest tile that is tested first.
-constexpr int ZTILE_DENSE = 128;
+// Which draws that can be tested first are, and by how many threads a tile:
+// the measurements are at k_zshade.
+constexpr int ZTILES_DIRECT = 2304, ZTILES_FEW = 512;
+constexpr int64_t ZPRIMS_DIRECT = 2048;
+constexpr int ZTILE_DENSE = 128, ZTILE_SPARSE = 16;  // raster triangles a tile
 constexpr int64_t ZDENSE_PIX = 512 * 1024;
 constexpr int ZTILE_PIX = 2048;
+enum ZPick : int32_t {
+    ZPICK_NONE,
+    ZPICK_DEVICE,  // both ways are launched; k_frag_scan picks one
+    ZPICK_CROWD,   // k_zshade leaves a draw with a crowded tile to the host, which has it shaded first
+};
 constexpr int SPAN_THREADS = 256;
 constexpr int SPAN_GROUP = 64;  // pairs whose spans are placed together
 // Spans per fragment-count block: the shading kernel's waves each take one
@@ -129,7 +137,7 @@ enum DrawStage : int {
     ST_FRAG_SCAN,
     ST_SHADE,
     ST_ROP,
-    ST_ZSHADE,  // in the place of the three before it, or after them (DrawArgs::zmode, zpick)
+    ST_ZSHADE,  // in the place of the three before it (DrawArgs::zmode)
     ST_COUNT
 };
 

@@ -377,6 +377,12 @@ FGL_D void spans_body(const DrawArgs &a, const G &g) {
     const uint32_t step = share ? g.nblk() : g.nblk() * WAVES;
     const int slot = share ? 0 : wave;
     uint64_t frags = 0;
+    // pairs of one tile that make it crowded, by the spans a pair has on average
+    uint32_t crowd = E;
+    if (a.zpick && NS) {
+        const uint64_t pairs = (uint64_t)max(a.crowd_min, NS / a.crowd_part) * E / NS;
+        crowd = pairs < E ? (uint32_t)pairs : E;
+    }
     for (uint32_t grp = first; grp < ngroups; grp += step) {
         const uint32_t p = grp * SPAN_GROUP + (uint32_t)lane;
         const uint32_t n = p < E ? a.pspans[p] : 0u;
@@ -394,6 +400,7 @@ FGL_D void spans_body(const DrawArgs &a, const G &g) {
             if (p < E) {
                 // the first and the last pair of a tile bound its spans
                 const uint32_t t = keys[p];
+                if (lane == 0 && crowd < E - p && keys[p + crowd] == t) a.ctr->crowded = 1u;
                 if (p == 0 || keys[p - 1] != t) a.tstart[t] = (uint32_t)(gbase + excl);
                 if (p + 1 == E || keys[p + 1] != t) a.tend[t] = (uint32_t)(gbase + excl) + n;
             }

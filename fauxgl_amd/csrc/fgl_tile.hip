@@ -367,12 +367,12 @@ template <class G>
 FGL_D void frag_scan_body(const DrawArgs &a, const G &grid) {
     __shared__ uint64_t wsum[FRAG_GROUP / 64];
     if (a.ctr->overflow) return;
-    if (a.zpick) {
-        // depth first, or not: two fragments a pixel (see k_zshade)
+    if (a.zpick == ZPICK_DEVICE) {
+        // depth first, or not: two fragments a pixel, no crowded tile (see k_zshade)
         const int l = threadIdx.x & 63;
         uint64_t all = a.ctr->ftot[l];
         for (int off = 32; off > 0; off >>= 1) all += __shfl_xor(all, off);
-        const bool zfirst = all >= 2ull * (uint64_t)a.W * (uint64_t)a.H;
+        const bool zfirst = all >= 2ull * (uint64_t)a.W * (uint64_t)a.H && !a.ctr->crowded;
         if (grid.bid() == 0 && threadIdx.x == 0) a.ctr->zfirst = zfirst ? 1u : 0u;
         if (zfirst) return;
     }
@@ -867,27 +867,48 @@ FGL_DRAW_KERNELS(k_rop, rop_body, __launch_bounds__(TILE_THREADS, FGL_ROP_WAVES)
 // tile's spans, their triangles' records, the shading inputs), some 2.5 us a
 // step under load, which the few workgroups whose tiles fit a CU's LDS hide
 // less well than k_shade's and k_rop's many waves do; with heavy overdraw, the
-// depth recurrence.  Measured against k_frag_scan + k_shade + k_rop: textured
-// soup at 1080p 0.80 against 1.85 ms, a sphere and a cube at 512x512 21
-// against 56 us, a cube at 64x64 12 against 35, the 871,306-triangle mesh at
-// 1080p 54 against 61; but the same mesh at 7680x4320 0.54 against 0.48 ms
-// and its 4096x4096 depth map 0.20 against 0.15, where each pixel has half a
-// fragment.  So draws of at most ZTILES_DIRECT tiles take it as they are, and
-// of larger ones those with two fragments a pixel or more, which k_frag_scan
-// finds out on the device (DrawArgs::zpick).  The device also picks for draws
-// of more than ZTILE_DENSE primitives a tile, whose spans of a pixel or two
-// leave each fragment a load of its own: whole draws at 1024x1024 of 871,306
-// triangles 311 us tested first, 289 picked; of 400,000 231 and 228; but of
-// 155,000 213 and 215, of 20,000 157 and 158.  In frames of at most ZDENSE_PIX
-// pixels the two differ by less than 4 us at any density.  Tiles of more than
-// ZTILE_PIX pixels leave one workgroup a CU, and too few at that: the 871,306
-// triangles at 1080p 198 us in 128x64 tiles and 109 in 64x64, against 61; a
-// sphere and a cube 110 and 67.  They are shaded first.
+// depth recurrence; where the spans crowd into few tiles, the one workgroup
+// that walks the fullest, while k_shade deals its fragments over the GPU.
 //
-// Sizes: the tile's depths, owners and colors (16 B a pixel) fill the LDS of
-// a CU with few workgroups, so a larger tile gets more threads; a draw of at
-// most ZTILES_FEW tiles leaves CUs idle and takes twice the threads a tile,
-// with shorter round sets (sphere and cube 33 -> 21 us).
+// Which draws take it (draw_zpick).  Figures are whole draws (clears, draw,
+// wait) in us, shaded first / tested first; the kernels alone on the textured
+// soup of 200,000 triangles at 1080p take 1850 / 800.
+//
+// - Up to ZPRIMS_DIRECT raster triangles all that can be: a cube at 128x128
+//   129 / 96, 600 triangles as a soup at 1080p 254 / 188, as a sphere 209 / 166;
+//   2000 crammed into 32x32 pixels of that frame 324 / 321, blended 344 / 393.
+// - Of more triangles, up to ZTILES_DIRECT tiles, those without a crowded
+//   tile: a sphere and a cube at 512x512 176 / 143, 20,000 triangles at
+//   1080p 215 / 194, on five tiles of 512x512 83 / 77; but 100,000 in 32x32
+//   pixels of 512x512 577 / 786, blended 624 / 971.  k_spans finds the crowd;
+//   k_zshade then draws nothing, and the host, which reads the counters
+//   anyway, launches the other way: 20 us more than at once, where launching
+//   both for the device to pick costs every draw that is tested 5 to 13.  So
+//   a crowd is what loses more than that: 10,000 spans (fullest tile 9164: 201
+//   / 207, 17,029: 239 / 282), if blended, whose survivors the tile's workgroup
+//   shades too, 5000 (4254: 208 / 236, 9164: 216 / 263), that are more than one
+//   in 32 of all, or 64 (soups, one in 55 opaque 487 / 451, one in 9 382 / 421;
+//   blended in 55 492 / 527, in 144 654 / 571).  With 256 threads a tile half
+//   of these.
+// - Above ZTILES_DIRECT tiles, and ZTILE_DENSE triangles a tile in frames of
+//   more than ZDENSE_PIX pixels, both ways are launched and k_frag_scan picks:
+//   tested first with two fragments a pixel or more and no tile with 1280 spans
+//   that are one in 256 (the soup at 2560x1440, one in 1700, 3594 / 1835).  The
+//   871,306-triangle mesh takes 366 / 384 at 3840x2160, 365 / 395 as a
+//   4096x4096 depth map, 216 / 214 as a 1400x1400 one: launching both costs 4.
+// - Tiles of more than ZTILE_PIX pixels leave one workgroup a CU, and too few
+//   at that (kernels: 871,306 triangles at 1080p 198 in 128x64 tiles and 109 in
+//   64x64, against 61).  They are shaded first.
+//
+// Threads a tile: its depths, owners and colors (16 B a pixel) fill the LDS
+// of a CU with few workgroups, so a tile of 2048 pixels gets 512.  Smaller ones
+// get them up to ZTILES_FEW tiles, where CUs are idle (sphere and cube at
+// 512x512, kernels 33 -> 21 us); above, opaque draws, few of whose tiles may
+// hold it all (256 -> 512 threads: 20,000 triangles on 67 tiles of a 1080p frame
+// 144 -> 132, the crammed 2000 421 -> 321; the soup unblended 985 -> 1002, at
+// 1023x767 835 -> 675),
+// and blended ones of up to ZTILE_SPARSE triangles a tile (8000: 285 -> 288; but
+// the soup 1241 -> 1359).
 template <int ZT>
 struct ZSize {
     static constexpr int B = ZT;                                                 // spans staged at a time
@@ -898,7 +919,6 @@ struct ZSize {
 };
 constexpr int ZT_MANY = TILE_PIX >= 2048 ? 512 : 256;
 constexpr int ZT_FEW = 512;
-constexpr int ZTILES_FEW = 512;
 // The color of the fragment of span `si` at tile pixel `pix`
 // (context.go:208-238 from the span's first pixel on, then the shader).
 template <int SH, class G>
@@ -941,7 +961,8 @@ FGL_D void zshade_body(const DrawArgs &a, const G &g) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     constexpr int WAVES = ZT / 64;
     __shared__ uint32_t again[3];  // some fragment of a round is still pending (in turn, zeroed a round ahead)
-    if (a.zpick && !a.ctr->zfirst) return;  // k_shade and k_rop draw it
+    // k_shade and k_rop draw it
+    if ((a.zpick == ZPICK_DEVICE && !a.ctr->zfirst) || (a.zpick == ZPICK_CROWD && a.ctr->crowded)) return;
     const int t = (int)g.bid();
     // (not the fragments' bit, which this launch may set: as in k_shade)
     const uint32_t overflow = a.ctr->overflow & ~OVF_FRAGS, s0 = a.tstart[t], s1 = a.tend[t];
@@ -1273,7 +1294,7 @@ static int zshade_variant(const DrawArgs &a) {
     }
 hipError_t launch_zshade(const DrawArgs &rep, hipStream_t s) {
     const dim3 grid(rep.ntiles);
-    if (rep.ntiles <= ZTILES_FEW) {
+    if (rep.z512) {
 #define FGL_LAUNCH(SH, BL) hipLaunchKernelGGL((k_zshade<SH, BL, ZT_FEW>), grid, dim3(ZT_FEW), 0, s, rep)
         FGL_ZSHADE_CASES(FGL_LAUNCH)
 #undef FGL_LAUNCH

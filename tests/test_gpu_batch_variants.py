@@ -132,8 +132,8 @@ def _deep(n, seed, extent):
 
 # (size, soup, shader, state, depth first): fragments tested before they are
 # shaded in every variant the others of a batch must not share a launch with
-# (color written or not, opaque or blended, the device's choice both ways), and
-# shaded first.  1600x1504 is 2350 tiles.  "shared" views follow each other on
+# (color written or not, opaque or blended, the device's choice both ways, a
+# crowded tile or none), and shaded first.  1600x1504 is 2350 tiles.  "shared" views follow each other on
 # one context, "empty" is a view without primitives.
 TESTED = [
     ((97, 67), "small", "phong", {}, True),
@@ -147,6 +147,11 @@ TESTED = [
     ((1600, 1504), "deep", "blend", {}, True),
     ((1600, 1504), "shallow", "blend", {}, False),
     ((1600, 1504), "deep", "phong", {"WriteColor": False}, True),
+    ((256, 256), "crowd", "phong", {}, False),
+    ((256, 256), "crowd", "blend", {}, False),
+    ((256, 256), "spread", "phong", {}, True),
+    ("shared", "spread", "phong", {}, True),
+    ("shared", "crowd", "phong", {}, False),
     ("shared", "small", "discard", {}, False),
     ("shared", "large", "solid", {}, True),
     ("shared", "small", "blend", {"WriteColor": False}, True),
@@ -157,10 +162,11 @@ TESTED = [
 def test_tested_first_equals_the_oracle(empty):
     import oracle as O
     from helpers import compare, oracle_shader
+    from test_gpu_depth_first import _crowd
     _say(f"batch of draws tested first and not, graph {empty}, 4 runs")
     home = A.NewContext(8, 8)
     soups = {"small": _deep(60, 1, 0.6), "large": _deep(400, 2, 0.3), "deep": _deep(60, 4, 0.9),
-             "shallow": _deep(40, 5, 0.1)}
+             "shallow": _deep(40, 5, 0.1), "spread": _deep(2500, 6, 0.05), "crowd": _crowd(2500, 256, 256, 32, 28)}
     light, eye = A.V(0.2, 0.4, 1).Normalize(), A.V(0, 0, 3)
     shaders = {"phong": A.PhongShader(A.Identity(), light, eye, A.Color(0.3, 0.6, 0.4, 1.0)),
                "blend": A.PhongShader(A.Identity(), light, eye, A.Color(0.3, 0.6, 0.4, 0.4)),

@@ -2,10 +2,11 @@
 against the oracle (color, depth, RasterizeInfo), over what selects and ends
 that path: opaque and blending colors of every shader, textures with and
 without a texel of alpha 0, color, depth write and depth test off, depth
-biases, marked clears before and after; few tiles (more threads a tile), many,
-and more than 2304 (the device decides by the fragments per pixel: the scenes
-have either side of two); every tile shape; overlap deep enough that the queue
-of blended survivors fills and wraps."""
+biases, marked clears before and after; few tiles, many, and more than 2304;
+draws of more than 2048 triangles, where the device picks, on both sides of
+what it picks by; every tile shape; overlap deep enough that the queue of
+blended survivors fills and wraps.  Every test says which way each draw is to
+have gone."""
 import numpy as np
 import pytest
 
@@ -129,22 +130,107 @@ def test_tile_shapes(shader, tile):
 @pytest.mark.parametrize("deep", [True, False])
 def test_many_tiles(shader, size, deep):
     W, H = size
-    prims = _soup(60, 4, 0.9) if deep else _soup(40, 5, 0.1)
+    prims = _soup(60, 4, 0.9) if deep else _soup(40, 5, 0.1)  # up to 2304 tiles not asked
     ctx = _check(f"{shader}, {W}x{H}, deep {deep}", SHADERS[shader](), W, H, [prims], [{}])
     assert (ctx.DrawStats()["fragments"] >= 2 * W * H) == deep
     assert ctx.DepthFirst() == (deep or W * H < 2304 * 1024)
 
 
+def _pad(prims, n):
+    """The triangles and as many with no pixel as make n."""
+    k = n - len(prims.position)
+    far = np.broadcast_to(np.array([[3.0, 0, 0], [4, 0, 0], [3, 1, 0]]), (k, 3, 3))
+    return A.Prims(np.concatenate([prims.position, far]), np.concatenate([prims.normal, M.with_face_normals(far)]),
+                   np.concatenate([prims.texture, np.zeros((k, 3, 2))]))
+
+
+def _quads(k):
+    """k screens of two triangles, behind each other in turns: 32 to 128 spans a
+    screen in a 32 x 32 tile (the box's last column wraps into the next row)."""
+    z = np.random.Generator(np.random.PCG64(k)).permutation(np.linspace(-0.9, 0.9, k))
+    a = np.array([[[-1, -1], [1, -1], [1, 1]], [[-1, -1], [1, 1], [-1, 1]]], dtype=float)
+    pos = np.concatenate([np.broadcast_to(a, (k, 2, 3, 2)), np.broadcast_to(z[:, None, None, None], (k, 2, 3, 1))], axis=3)
+    pos = np.ascontiguousarray(pos.reshape(-1, 3, 3))
+    return A.Prims(pos, M.with_face_normals(pos), np.random.Generator(np.random.PCG64(1)).uniform(0, 1, (2 * k, 3, 2)))
+
+
+def _crowd(n, W, H, px=32, size=8):
+    """n triangles of some `size` pixels in the frame's first px x px."""
+    p = _soup(n, 12, 1.0)
+    c = p.position.mean(axis=1, keepdims=True)
+    pos = c + (p.position - c) * [size / px, size / px, 0.1]
+    pos = np.clip(pos, -1, 1) * [px / W, px / H, 1] + [px / W - 1, 1 - px / H, 0]
+    return A.Prims(pos, M.with_face_normals(pos), p.texture)
+
+
+# (frame, draw, shader, tested first).  A tile is 32 x 32.  Draws of more than
+# 2048 triangles are tested first unless a tile is crowded: it holds more than
+# 10,000 spans and more than a 32nd of all (blended 5000 and a 64th; in
+# more than 512 tiles, with more than 16 triangles a tile, 2500 and a 128th).
+# Above 2304 tiles, and 128 triangles a tile in a large frame, they are where
+# there are two fragments a pixel and no tile has 1280 spans and a 256th.
+PICKS = {
+    "crowd, the largest unasked": ((1920, 1080), lambda W, H: _crowd(2048, W, H, 32, 28), "phong", True),
+    "crowd": ((1920, 1080), lambda W, H: _crowd(2500, W, H, 32, 28), "phong", False),
+    "no crowd": ((1920, 1080), lambda W, H: _crowd(2500, W, H, 320, 8), "phong", True),
+    "crowd, blended": ((1920, 1080), lambda W, H: _crowd(2200, W, H, 32, 11), "phong translucent", False),
+    "the same, opaque": ((1920, 1080), lambda W, H: _crowd(2200, W, H, 32, 11), "phong", True),
+    "crowd, few tiles": ((256, 256), lambda W, H: _crowd(2500, W, H, 32, 28), "phong", False),
+    "crowd, one tile": ((32, 32), lambda W, H: _quads(450), "texture", False),
+    "few tiles, short": ((96, 64), lambda W, H: _quads(45), "phong", True),
+    "few tiles, uneven": ((256, 64), lambda W, H: _quads(350), "solid", False),
+    "few tiles, even": ((1024, 128), lambda W, H: _quads(350), "solid", True),
+    "few tiles, blended, uneven": ((512, 64), lambda W, H: _quads(180), "solid translucent", False),
+    "few tiles, blended, even": ((1024, 256), lambda W, H: _quads(180), "solid translucent", True),
+    "many triangles, blended, crowd": ((864, 640), lambda W, H: _pad(_crowd(1000, W, H, 32, 12), 8641), "texture", False),
+    "not so many, blended": ((864, 640), lambda W, H: _pad(_crowd(1000, W, H, 32, 12), 8640), "texture", True),
+    "dense, shallow": ((1000, 800), lambda W, H: _soup(102401, 6, 0.004), "phong", False),
+    "not so dense": ((1000, 800), lambda W, H: _soup(102400, 6, 0.004), "phong", True),
+    "dense, deep": ((1000, 800), lambda W, H: _soup(102401, 6, 0.03), "phong", True),
+    "dense, deep, crowded": ((1000, 800), lambda W, H: _pad(_crowd(4000, W, H, 200, 190), 102401), "phong", False),
+    "many tiles, deep": ((1600, 1504), lambda W, H: _quads(6), "phong", True),
+    "many tiles, shallow": ((1600, 1504), lambda W, H: _quads(1), "phong", False),
+    "many tiles, deep, no color": ((1600, 1504), lambda W, H: _quads(6), "solid", True),
+    "many tiles, deep, crowded": ((1600, 1504), lambda W, H: _crowd(6000, W, H, 200, 190), "phong", False),
+}
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", [102400, 102401])
-@pytest.mark.parametrize("deep", [True, False])
-def test_dense_triangles(n, deep):
-    # 800 tiles: at 128 triangles a tile depth first, above it the device picks
-    W, H = 1000, 800
-    prims = _soup(n, 6, 0.03 if deep else 0.004)
-    ctx = _check(f"{n} triangles, deep {deep}", SHADERS["phong"](), W, H, [prims], [{}])
-    assert (ctx.DrawStats()["fragments"] >= 2 * W * H) == deep
-    assert ctx.DepthFirst() == (deep or n == 102400)
+@pytest.mark.parametrize("name", list(PICKS))
+def test_picks(name):
+    (W, H), draw, shader, want = PICKS[name]
+    prims = draw(W, H)
+    if len(prims.position) < 2048:
+        prims = _pad(prims, 2049)
+    state = {"WriteColor": False} if name.endswith("no color") else {}
+    ctx = _check(name, SHADERS[shader](), W, H, [prims], [state], first=lambda st: want)
+    deep = ctx.DrawStats()["fragments"] >= 2 * W * H
+    assert deep or ", deep" not in name
+    assert ctx.DrawStats()["reruns"] == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,want", [(1024, True), (1300, False)])
+def test_picks_lines(n, want):
+    """A line is two triangles to the rule."""
+    W, H = 640, 480
+    _say(f"depth first: {n} lines")
+    p = _crowd(n, W, H, 32, 30).position[:, :2].copy()
+    lines = A.Prims(p, None, None, None, nv=2)
+    sh = SHADERS["solid"]()
+    octx, ctx = O.Context(W, H), A.NewContext(W, H)
+    octx.clear_color(tuple(A.White))
+    octx.clear_depth(A.MaxFloat64)
+    ctx.ClearColorBufferWith(A.White)
+    octx.set_shader(oracle_shader(sh))
+    octx.set_state(O.make_state(front_face=O.FACE_CCW, line_width=2.0, read_depth=True, write_depth=True,
+                                write_color=True, alpha_blend=True, wireframe=False, cull=O.CULL_BACK, depth_bias=0.0))
+    ctx.Shader = sh
+    ri = octx.draw_lines(O.Mesh(lines=lines.arrays()), 1)
+    gi = tuple(ctx.DrawLines(lines))
+    assert ctx.DepthFirst() == want
+    res = compare((octx.color(), octx.depth(), [ri]), (ctx.Image(), ctx.DepthBuffer, [gi]), color_tol=0)
+    assert res["ok"], res
 
 
 @pytest.mark.gpu
@@ -183,3 +269,28 @@ def test_forced_fragment_overflow(shader, size, n):
         assert ctx.DepthFirst() == (shader != "texture with a hole")
         res = compare((octx.color(), octx.depth(), ri), (ctx.Image(), ctx.DepthBuffer, gi), color_tol=0)
         assert res["ok"], res
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("caps", [{"fragments": 1}, {"spans": 1}, {"pairs": 1}, {"spans": 1, "fragments": 1}])
+def test_forced_overflow_of_a_crowd(caps):
+    """A draw that a crowded tile sends the other way, and that runs out on it."""
+    W, H = 256, 256
+    _say(f"depth first: crowd, forced {caps}")
+    prims, sh = _crowd(2500, W, H, 32, 28), SHADERS["phong translucent"]()
+    octx, ctx = O.Context(W, H), A.NewContext(W, H)
+    ctx.Cull, ctx.Shader = A.CullNone, sh
+    octx.clear_color(tuple(A.White))
+    octx.clear_depth(A.MaxFloat64)
+    octx.set_shader(oracle_shader(sh))
+    octx.set_state(O.make_state(front_face=O.FACE_CCW, line_width=2.0, read_depth=True, write_depth=True,
+                                write_color=True, alpha_blend=True, wireframe=False, cull=A.CullNone, depth_bias=0.0))
+    ctx.DrawTriangles(prims)  # sizes the buffers
+    ctx.ClearColorBufferWith(A.White)
+    ctx.ClearDepthBuffer()
+    ri = octx.draw_triangles(O.Mesh(tris=prims.arrays()), 1)
+    ctx.ForceCapacities(**caps)
+    gi = tuple(ctx.DrawTriangles(prims))
+    assert ctx.DrawStats()["reruns"] == 1 and not ctx.DepthFirst()
+    res = compare((octx.color(), octx.depth(), [ri]), (ctx.Image(), ctx.DepthBuffer, [gi]), color_tol=0)
+    assert res["ok"], res
