@@ -417,6 +417,8 @@ struct fgl_ctx {
     DevBuf dpart, dimg;
     DevBuf png;    // the size and checksums of EncodePNG's stream
     HostBuf hpng;  // the same as the host reads them back
+    DevBuf texflag;    // whether the last texture has a texel of alpha 0
+    HostBuf htexflag;
     uint32_t side_rec_cap = 0, side_vtx_cap = 0, pair_cap = 0;
     DrawCounters last{};
 
@@ -671,6 +673,20 @@ int fill_shader(fgl_ctx *c, const fgl_shader *sh, DevShader &d) {
 }
 
 constexpr int64_t kMaxPrims = (int64_t)1 << 26;
+// Texels up to which the host looks for alphas of 0 itself.
+constexpr size_t kHostTexels = (size_t)1 << 18;
+
+// no texel (a T, the alpha in its top quarter) of alpha 0
+template <class T>
+bool no_hole(const void *texels, size_t n) {
+    T hole = 0;
+    for (size_t k = 0; k < n; k++) {
+        T t;
+        std::memcpy(&t, static_cast<const uint8_t *>(texels) + k * sizeof(T), sizeof(T));
+        hole |= (t >> (6 * sizeof(T))) == 0;
+    }
+    return !hole;
+}
 // Side vertices (from clipping) per draw; keeps the shading kernels'
 // attribute offsets within 32 bits.
 constexpr uint64_t kMaxSideVtx = (uint64_t)1 << 28;
@@ -1251,17 +1267,27 @@ int fgl_texture_create(fgl_ctx *ctx, int32_t width, int32_t height, int32_t kind
     t.w = width;
     t.h = height;
     t.kind = kind;
-    t.solid = true;
-    const size_t ntexel = (size_t)width * height;
-    if (kind == FGL_TEX_RGBA16) {
-        for (size_t k = 0; k < ntexel && t.solid; k++) t.solid = static_cast<const uint16_t *>(texels)[4 * k + 3] != 0;
-    } else {
-        for (size_t k = 0; k < ntexel && t.solid; k++) t.solid = static_cast<const uint8_t *>(texels)[4 * k + 3] != 0;
-    }
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return drop(e, "hipSetDevice");
     if ((e = t.d.ensure(bytes)) != hipSuccess) return drop(e, "texture allocation");
     if ((e = hipMemcpy(t.d.p, texels, bytes, hipMemcpyHostToDevice)) != hipSuccess) return drop(e, "texture upload");
+    // Where the alphas lie in the host's cache it looks itself; the device
+    // and a read back take 45 us (400x400 in 16 bits: by the host 18, by the device
+    // 45; byte by byte and one after another it took 0.24 ms at 1024x1024, 15 at
+    // 8192x8192).
+    const size_t ntexel = (size_t)width * height;
+    const bool wide = kind == FGL_TEX_RGBA16;
+    if (ntexel <= kHostTexels) {
+        t.solid = wide ? no_hole<uint64_t>(texels, ntexel) : no_hole<uint32_t>(texels, ntexel);
+    } else {
+        if ((e = ctx->texflag.ensure(4)) != hipSuccess || (e = ctx->htexflag.ensure(4)) != hipSuccess ||
+            (e = hipMemsetAsync(ctx->texflag.p, 0, 4, ctx->stream)) != hipSuccess ||
+            (e = launch_tex_hole(t.d.p, (int64_t)ntexel, wide, ctx->texflag.as<uint32_t>(), ctx->stream)) != hipSuccess ||
+            (e = hipMemcpyAsync(ctx->htexflag.p, ctx->texflag.p, 4, hipMemcpyDeviceToHost, ctx->stream)) != hipSuccess ||
+            (e = wait_stream(ctx->stream)) != hipSuccess)
+            return drop(e, "texture scan");
+        t.solid = *ctx->htexflag.as<uint32_t>() == 0;
+    }
     ctx->next_tex++;
     *handle = h;
     return FGL_OK;

@@ -256,6 +256,8 @@ hipError_t launch_resolve(const uint32_t *src, int32_t sw, int32_t sh, uint32_t 
                           int32_t dh, int32_t filter, const int16_t *wx, const int32_t *ox, int32_t flx,
                           const int16_t *wy, const int32_t *oy, int32_t fly, const ResolveTent4 &t4,
                           const uint8_t *cblk, int32_t cbw, uint32_t clear_color, hipStream_t s);
+// flag[0] = 1 where one of n texels (wide: 16 bits a channel) has alpha 0
+hipError_t launch_tex_hole(const void *texels, int64_t n, bool wide, uint32_t *flag, hipStream_t s);
 hipError_t launch_depth_minmax(const double *depth, int64_t n, double *partial, int32_t nblocks, hipStream_t s);
 hipError_t launch_depth_image(const double *depth, int64_t n, const double *partial, int32_t nblocks,
                               uint16_t *out, hipStream_t s);

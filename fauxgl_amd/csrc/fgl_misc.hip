@@ -558,6 +558,31 @@ hipError_t launch_resolve(const uint32_t *src, int32_t sw, int32_t sh, uint32_t 
 // DepthImage (context.go:87-117): lo/hi over depths != MaxFloat64, then
 // uint16(t * 0xffff) with t = (d - lo) / (hi - lo) (t = 1 for cleared).
 
+// ---------------------------------------------------------------------------
+// whether a texture has a texel of alpha 0: flag[0] = 1 (every writer stores
+// the same value).  words: the texels, one (8 bits a channel) or two words
+// each, alpha in the top bits of the (second) word.
+template <bool WIDE>
+__global__ __launch_bounds__(256) void k_tex_hole(const uint32_t *words, int64_t nwords, uint32_t *flag) {
+    auto hole = [](uint32_t w) { return (w >> (WIDE ? 16 : 24)) == 0; };
+    const int64_t n4 = nwords / 4, t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    bool seen = false;
+    for (int64_t i = t0; i < n4; i += (int64_t)gridDim.x * blockDim.x) {
+        const uint4 v = reinterpret_cast<const uint4 *>(words)[i];
+        seen |= hole(v.y) || hole(v.w) || (!WIDE && (hole(v.x) || hole(v.z)));
+    }
+    const int64_t rest = 4 * n4 + t0;  // the last texels, below one load
+    if (rest < nwords && (!WIDE || (rest & 1))) seen |= hole(words[rest]);
+    if (__ballot(seen) != 0 && (threadIdx.x & 63) == 0) flag[0] = 1u;
+}
+hipError_t launch_tex_hole(const void *texels, int64_t n, bool wide, uint32_t *flag, hipStream_t s) {
+    const int64_t nwords = wide ? 2 * n : n;
+    const dim3 grid(grid_for((nwords + 3) / 4));
+    if (wide) hipLaunchKernelGGL(k_tex_hole<true>, grid, dim3(256), 0, s, static_cast<const uint32_t *>(texels), nwords, flag);
+    else hipLaunchKernelGGL(k_tex_hole<false>, grid, dim3(256), 0, s, static_cast<const uint32_t *>(texels), nwords, flag);
+    return hipGetLastError();
+}
+
 constexpr double kMaxFloat64 = 1.79769313486231570814527423731704356798070e+308;
 
 // Four loads of two depths in flight per thread: one depth at a time left
