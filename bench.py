@@ -436,8 +436,8 @@ def kernel_roofline(name, avg_ms, stats, W, H, ssaa, shader="phong"):
         nbytes = 4 * npix + 4 * W * H
         unit_desc = f"4 B x {npix} source pixels + 4 B x {W * H} resolved pixels"
     elif name == "zshade":
-        # shades only what its depth tests leave: bounded from below by the
-        # spans it reads and the pixels it writes
+        # shades only what its depth tests leave; counts every pixel of the
+        # frame as written, which tiles without a fragment are not
         nbytes = 32 * stats["spans"] + 12 * npix
         unit_desc = f"32 B x {stats['spans']} spans read + 12 B x {npix} pixels written"
     elif name == "spans":

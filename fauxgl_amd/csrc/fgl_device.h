@@ -100,7 +100,6 @@ struct DevShader {
 struct DevState {
     int32_t read_depth, write_depth, write_color, alpha_blend, wireframe;
     int32_t front_face, cull;
-    int32_t early_z;  // early depth reject before shading is exact (see tile kernel)
     double line_width, depth_bias;
 };
 

@@ -785,9 +785,6 @@ void draw_setup(fgl_ctx *c, const fgl_state *st, const TileOps &T, int kind, con
     a.st.cull = st->cull;
     a.st.line_width = st->line_width;
     a.st.depth_bias = st->depth_bias;
-    // Rejecting bz > depth before shading equals the reference's locked test
-    // only while stored depth cannot increase.
-    a.st.early_z = a.st.read_depth && (!a.st.write_depth || st->depth_bias >= 0);
     screen_matrix(c->W, c->H, a.S);
     a.color = c->color.as<uint32_t>();
     a.depth = c->depth.as<double>();
