@@ -631,8 +631,8 @@ __global__ __launch_bounds__(256) void k_depth_minmax(const double *depth, int64
 }
 
 // Each workgroup first reduces the partials together.  (Every thread walking
-// all 512 of them by itself was most of the kernel: 378 us of 4096 x 4096; now
-// 28.)
+// all 512 of them by itself was most of the kernel: 378 us of 4096 x 4096; with
+// the vector accesses now 28.)
 // VEC: four pixels a thread with 16- and 8-byte accesses; the launcher takes
 // it where the output allows.
 template <bool VEC>
