@@ -124,7 +124,7 @@ struct DrawCounters {
     // part wave % 64)
     unsigned long long ftot[64];
     uint32_t crowded;            // a tile holds too large a part of the spans (DrawArgs::crowd_min)
-    uint32_t pad3;
+    uint32_t crowd_pairs;        // pairs that make a tile so
 };
 constexpr int UPD_PARTS = 64;
 // DrawCounters::overflow: fragments past the capacity.  The kernels that find

@@ -129,6 +129,12 @@ FGL_D void span_scan_body(const DrawArgs &a, const G &) {
         a.ctr->nspans = total > a.span_cap ? a.span_cap : (uint32_t)total;
         a.ctr->spans_lo = (uint32_t)total;
         a.ctr->spans_hi = (uint32_t)(total >> 32);
+        if (a.zpick) {
+            // pairs of one tile that make it crowded, by the spans a pair has on average
+            const uint64_t spans = max((uint64_t)a.crowd_min, total / a.crowd_part);
+            const uint64_t pairs = total ? spans * E / total : E;
+            a.ctr->crowd_pairs = pairs < E ? (uint32_t)pairs : E;
+        }
     }
 }
 FGL_DRAW_KERNELS(k_span_scan, span_scan_body, __launch_bounds__(SCAN_THREADS))
@@ -377,12 +383,7 @@ FGL_D void spans_body(const DrawArgs &a, const G &g) {
     const uint32_t step = share ? g.nblk() : g.nblk() * WAVES;
     const int slot = share ? 0 : wave;
     uint64_t frags = 0;
-    // pairs of one tile that make it crowded, by the spans a pair has on average
-    uint32_t crowd = E;
-    if (a.zpick && NS) {
-        const uint64_t pairs = (uint64_t)max(a.crowd_min, NS / a.crowd_part) * E / NS;
-        crowd = pairs < E ? (uint32_t)pairs : E;
-    }
+    const uint32_t crowd = a.zpick ? a.ctr->crowd_pairs : E;
     for (uint32_t grp = first; grp < ngroups; grp += step) {
         const uint32_t p = grp * SPAN_GROUP + (uint32_t)lane;
         const uint32_t n = p < E ? a.pspans[p] : 0u;
