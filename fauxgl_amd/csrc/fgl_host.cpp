@@ -827,16 +827,16 @@ void draw_zpick(DrawArgs &a, int kind, const bool *picked) {
     const bool few = a.ntiles <= ZTILES_FEW;
     const bool large = a.ntiles > ZTILES_DIRECT ||
                        ((int64_t)a.W * a.H > ZDENSE_PIX && n > (int64_t)ZTILE_DENSE * a.ntiles);
-    a.z512 = few || (!large && (a.zmode == 1 || n <= (int64_t)ZTILE_SPARSE * a.ntiles));
+    a.z512 = few || (!large && (a.zmode == 1 || n <= ZPRIMS_DIRECT));
     if (large) {
         a.zpick = ZPICK_DEVICE;
         a.crowd_min = 1280;
         a.crowd_part = 256;
     } else if (n > ZPRIMS_DIRECT) {
         a.zpick = ZPICK_CROWD;
-        const uint32_t f = (a.zmode == 2 ? 2 : 1) * (a.z512 ? 1 : 2);
-        a.crowd_min = 10000 / f;
-        a.crowd_part = 32 * f;
+        const bool blend = a.zmode == 2;
+        a.crowd_min = (blend ? 3500 : 6000) / (a.z512 ? 1 : 2);
+        a.crowd_part = (blend ? 64 : 32) * (a.z512 ? 1 : 2);
     }
     if (a.zpick && picked) {
         a.zpick = ZPICK_NONE;

@@ -104,7 +104,7 @@ constexpr int VS_THREADS = 256;
 // the measurements are at k_zshade.
 constexpr int ZTILES_DIRECT = 2304, ZTILES_FEW = 512;
 constexpr int64_t ZPRIMS_DIRECT = 2048;
-constexpr int ZTILE_DENSE = 128, ZTILE_SPARSE = 16;  // raster triangles a tile
+constexpr int ZTILE_DENSE = 128;  // raster triangles a tile
 constexpr int64_t ZDENSE_PIX = 512 * 1024;
 constexpr int ZTILE_PIX = 2048;
 enum ZPick : int32_t {

@@ -884,12 +884,12 @@ FGL_DRAW_KERNELS(k_rop, rop_body, __launch_bounds__(TILE_THREADS, FGL_ROP_WAVES)
 //   k_zshade then draws nothing, and the host, which reads the counters
 //   anyway, launches the other way: 20 us more than at once, where launching
 //   both for the device to pick costs every draw that is tested 5 to 13.  So
-//   a crowd is what loses more than that: 10,000 spans (fullest tile 9164: 201
-//   / 207, 17,029: 239 / 282), if blended, whose survivors the tile's workgroup
-//   shades too, 5000 (4254: 208 / 236, 9164: 216 / 263), that are more than one
-//   in 32 of all, or 64 (soups, one in 55 opaque 487 / 451, one in 9 382 / 421;
-//   blended in 55 492 / 527, in 144 654 / 571).  With 256 threads a tile half
-//   of these.
+//   a crowd is what loses about that: 6000 spans (fullest tile 3733: 124 / 127,
+//   6319: 152 / 178, 17,029: 239 / 282), if blended, whose survivors the tile's
+//   workgroup shades too, 3500 (3121: 183 / 192, 4117: 156 / 186, 9164: 216 /
+//   263), that are more than one in 32 of all, or 64 (soups, one in 55 opaque
+//   487 / 451, one in 9 382 / 421; blended in 55 492 / 527, in 144 654 / 571).
+//   With 256 threads a tile half of these.
 // - Above ZTILES_DIRECT tiles, and ZTILE_DENSE triangles a tile in frames of
 //   more than ZDENSE_PIX pixels, both ways are launched and k_frag_scan picks:
 //   tested first with two fragments a pixel or more and no tile with 1280 spans
@@ -906,9 +906,8 @@ FGL_DRAW_KERNELS(k_rop, rop_body, __launch_bounds__(TILE_THREADS, FGL_ROP_WAVES)
 // 512x512, kernels 33 -> 21 us); above, opaque draws, few of whose tiles may
 // hold it all (256 -> 512 threads: 20,000 triangles on 67 tiles of a 1080p frame
 // 144 -> 132, the crammed 2000 421 -> 321; the soup unblended 985 -> 1002, at
-// 1023x767 835 -> 675),
-// and blended ones of up to ZTILE_SPARSE triangles a tile (8000: 285 -> 288; but
-// the soup 1241 -> 1359).
+// 1023x767 835 -> 675), and blended ones that are not asked (the crammed 2000
+// 495 -> 393; but the soup 1241 -> 1359, one of 30,000 433 -> 458).
 template <int ZT>
 struct ZSize {
     static constexpr int B = ZT;                                                 // spans staged at a time

@@ -165,25 +165,27 @@ def _crowd(n, W, H, px=32, size=8):
 
 # (frame, draw, shader, tested first).  A tile is 32 x 32.  Draws of more than
 # 2048 triangles are tested first unless a tile is crowded: it holds more than
-# 10,000 spans and more than a 32nd of all (blended 5000 and a 64th; in
-# more than 512 tiles, with more than 16 triangles a tile, 2500 and a 128th).
+# 6000 spans and more than a 32nd of all (blended 3500 and a 64th; in
+# more than 512 tiles 1750 and a 128th).
 # Above 2304 tiles, and 128 triangles a tile in a large frame, they are where
 # there are two fragments a pixel and no tile has 1280 spans and a 256th.
 PICKS = {
     "crowd, the largest unasked": ((1920, 1080), lambda W, H: _crowd(2048, W, H, 32, 28), "phong", True),
     "crowd": ((1920, 1080), lambda W, H: _crowd(2500, W, H, 32, 28), "phong", False),
     "no crowd": ((1920, 1080), lambda W, H: _crowd(2500, W, H, 320, 8), "phong", True),
-    "crowd, blended": ((1920, 1080), lambda W, H: _crowd(2200, W, H, 32, 11), "phong translucent", False),
-    "the same, opaque": ((1920, 1080), lambda W, H: _crowd(2200, W, H, 32, 11), "phong", True),
+    "crowd, blended": ((1920, 1080), lambda W, H: _crowd(2200, W, H, 32, 8), "phong translucent", False),
+    "the same, opaque": ((1920, 1080), lambda W, H: _crowd(2200, W, H, 32, 8), "phong", True),
     "crowd, few tiles": ((256, 256), lambda W, H: _crowd(2500, W, H, 32, 28), "phong", False),
     "crowd, one tile": ((32, 32), lambda W, H: _quads(450), "texture", False),
-    "few tiles, short": ((96, 64), lambda W, H: _quads(45), "phong", True),
+    "few tiles, short": ((96, 64), lambda W, H: _quads(40), "phong", True),
     "few tiles, uneven": ((256, 64), lambda W, H: _quads(350), "solid", False),
     "few tiles, even": ((1024, 128), lambda W, H: _quads(350), "solid", True),
     "few tiles, blended, uneven": ((512, 64), lambda W, H: _quads(180), "solid translucent", False),
     "few tiles, blended, even": ((1024, 256), lambda W, H: _quads(180), "solid translucent", True),
-    "many triangles, blended, crowd": ((864, 640), lambda W, H: _pad(_crowd(1000, W, H, 32, 12), 8641), "texture", False),
-    "not so many, blended": ((864, 640), lambda W, H: _pad(_crowd(1000, W, H, 32, 12), 8640), "texture", True),
+    "many tiles, blended, crowd": ((864, 640), lambda W, H: _crowd(1000, W, H, 32, 8), "texture", False),
+    "the same, opaque, many tiles": ((864, 640), lambda W, H: _crowd(1000, W, H, 32, 8), "phong", True),
+    "the same, few tiles": ((512, 512), lambda W, H: _crowd(1000, W, H, 32, 8), "texture", True),
+    "the same, not asked": ((864, 640), lambda W, H: _pad(_crowd(1000, W, H, 32, 8), 2048), "texture", True),
     "dense, shallow": ((1000, 800), lambda W, H: _soup(102401, 6, 0.004), "phong", False),
     "not so dense": ((1000, 800), lambda W, H: _soup(102400, 6, 0.004), "phong", True),
     "dense, deep": ((1000, 800), lambda W, H: _soup(102401, 6, 0.03), "phong", True),
