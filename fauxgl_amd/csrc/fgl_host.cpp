@@ -823,7 +823,8 @@ int draw_zmode(const DrawArgs &a) {
 // was tested first.
 void draw_zpick(DrawArgs &a, int kind, const bool *picked) {
     // raster triangles (a line is two, and wireframe draws three lines)
-    const int64_t n = a.in.n * (kind == PRIM_LINE ? 2 : a.st.wireframe ? 6 : 1);
+    const int per = kind == PRIM_LINE ? 2 : a.st.wireframe ? 6 : 1;
+    const int64_t n = a.in.n * per;
     const bool few = a.ntiles <= ZTILES_FEW;
     const bool large = a.ntiles > ZTILES_DIRECT ||
                        ((int64_t)a.W * a.H > ZDENSE_PIX && n > (int64_t)ZTILE_DENSE * a.ntiles);
@@ -832,7 +833,7 @@ void draw_zpick(DrawArgs &a, int kind, const bool *picked) {
         a.zpick = ZPICK_DEVICE;
         a.crowd_min = 1280;
         a.crowd_part = 256;
-    } else if (n > ZPRIMS_DIRECT) {
+    } else if (n > ZPRIMS_DIRECT && (per == 1 || !a.z512)) {
         a.zpick = ZPICK_CROWD;
         const bool blend = a.zmode == 2;
         a.crowd_min = (blend ? 3500 : 6000) / (a.z512 ? 1 : 2);

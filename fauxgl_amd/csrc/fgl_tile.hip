@@ -890,6 +890,13 @@ FGL_DRAW_KERNELS(k_rop, rop_body, __launch_bounds__(TILE_THREADS, FGL_ROP_WAVES)
 //   263), that are more than one in 32 of all, or 64 (soups, one in 55 opaque
 //   487 / 451, one in 9 382 / 421; blended in 55 492 / 527, in 144 654 / 571).
 //   With 256 threads a tile half of these.
+//   Lines and wireframes are not asked with 512: a mesh's follow each other
+//   over the same pixels, where k_rop's rounds conflict more (the wireframe of
+//   80,000 triangles at 160x120 4579 / 2934, as a speck at 512x512 25,900 /
+//   12,800; the edges of 20,000 drawn as lines 16,220 / 8060; 20,000 random
+//   ones at 104x293 318 / 293).  That costs thin triangles piled up in no order:
+//   20,000 lines in 32x32 pixels of 512x512 706 / 989, long ones in 100x100
+//   606 / 1298.
 // - Above ZTILES_DIRECT tiles, and ZTILE_DENSE triangles a tile in frames of
 //   more than ZDENSE_PIX pixels, both ways are launched and k_frag_scan picks:
 //   tested first with two fragments a pixel or more and no tile with 1280 spans

@@ -164,7 +164,7 @@ def _crowd(n, W, H, px=32, size=8):
 
 
 # (frame, draw, shader, tested first).  A tile is 32 x 32.  Draws of more than
-# 2048 triangles are tested first unless a tile is crowded: it holds more than
+# 2048 filled triangles are tested first unless a tile is crowded: it holds more than
 # 6000 spans and more than a 32nd of all (blended 3500 and a 64th; in
 # more than 512 tiles 1750 and a 128th).
 # Above 2304 tiles, and 128 triangles a tile in a large frame, they are where
@@ -211,15 +211,35 @@ def test_picks(name):
     assert ctx.DrawStats()["reruns"] == 0
 
 
+# lines and wireframe triangles in one tile, more than a crowd of filled
+# triangles: asked only where a tile gets 256 threads (blended, more than 512 tiles)
+SMALL, MANY = (640, 480), (864, 640)
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("n,want", [(1024, True), (1300, False)])
-def test_picks_lines(n, want):
+@pytest.mark.parametrize("size,shader,n,want", [(SMALL, "solid", 341, True), (SMALL, "solid", 500, True),
+                                                (SMALL, "solid translucent", 500, True), (MANY, "solid", 500, True),
+                                                (MANY, "solid translucent", 500, False),
+                                                (MANY, "solid translucent", 341, True)])
+def test_picks_wireframe(size, shader, n, want):
+    """A wireframe triangle is six to the rule."""
+    prims = _crowd(n, *size, 32, 28)
+    _check(f"{n} wireframe triangles, {shader}, {size}", SHADERS[shader](), *size, [prims], [{"Wireframe": True}],
+           first=lambda st: want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("size,shader,n,want", [(SMALL, "solid", 1024, True), (SMALL, "solid", 1300, True),
+                                                (SMALL, "solid translucent", 1300, True), (MANY, "solid", 1300, True),
+                                                (MANY, "solid translucent", 1300, False),
+                                                (MANY, "solid translucent", 1024, True)])
+def test_picks_lines(size, shader, n, want):
     """A line is two triangles to the rule."""
-    W, H = 640, 480
-    _say(f"depth first: {n} lines")
+    W, H = size
+    _say(f"depth first: {n} lines, {shader}, {W}x{H}")
     p = _crowd(n, W, H, 32, 30).position[:, :2].copy()
     lines = A.Prims(p, None, None, None, nv=2)
-    sh = SHADERS["solid"]()
+    sh = SHADERS[shader]()
     octx, ctx = O.Context(W, H), A.NewContext(W, H)
     octx.clear_color(tuple(A.White))
     octx.clear_depth(A.MaxFloat64)
